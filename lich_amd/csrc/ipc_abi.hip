@@ -648,8 +648,9 @@ bool narrow_eligible(int L, const int* dims, int storage, int operand, int split
   if (split == IPC_SPLIT_W) return false;  // the whole-step kernel carries split 1 or 3
   for (int l = 0; l < L; ++l)
     if (dims[l] > NARROW_MAX_WIDTH) return false;
-  // one column block's states, errors and staged activations must fit in LDS
-  return narrow_lds_bytes(dims, L, operand, split) <= NARROW_LDS_LIMIT - 1024;
+  // one column block's states, errors and staged activations must fit in LDS,
+  // next to the kernel's static copies of its arguments and layout
+  return narrow_lds_bytes(dims, L, operand, split) <= NARROW_LDS_LIMIT - NARROW_STATIC_LDS;
 }
 
 bool wide_eligible(int storage, int operand, int split, int wmode, int B) {

@@ -61,6 +61,10 @@ struct NarrowLds {
   int xr_bytes, ef_base, fs_base, es_base, outer_base, total;
 };
 
+// Static LDS of the kernel (its argument block and this layout) next to the
+// dynamic buffers.
+constexpr int NARROW_STATIC_LDS = ((int)(sizeof(NarrowArgs) + sizeof(NarrowLds)) + 15) / 16 * 16;
+
 __host__ __device__ inline int narrow_ldk(int d, int KS, int PAD) { return (d + KS - 1) / KS * KS + PAD; }
 
 __host__ __device__ inline void narrow_lds_layout(const int* dims, int L, int KS, int PAD, int esize, bool split3,

@@ -644,3 +644,24 @@ def test_dma_tile_ids_are_refused_where_the_dma_kernel_cannot_run():
         assert rc == nat.ERR_CONFIG and "LDS-DMA" in nat.last_error()
     assert lib.ipc_pred_err(P, P, P, P, 64, 64, 128, 1, nat.DT_BF16, nat.DT_BF16, 1, 2, nat.TILE_COUNT, None) == \
         nat.ERR_CONFIG
+
+
+@pytest.mark.parametrize("features,want", [(160, nat.PATH_NARROW), (208, nat.PATH_NARROW), (224, nat.PATH_PHASED),
+                                           (240, nat.PATH_PHASED)])
+def test_column_kernel_leaves_room_for_its_static_lds(features, want):
+    """A column block whose buffers fill the LDS up to the kernel's static
+    1,440 bytes could not be launched (the LDS limit was refused): such a net
+    takes the phased path."""
+    lib = nat.lib()
+    dims = (ctypes.c_int * 8)(10, 87, 87, 87, 87, 87, 87, features)
+    h = ctypes.c_void_p()
+    # layout restated: raw x, eps, f(x) and eps operands of 16 columns (fp32: rows of
+    # 16-padded contractions plus 4), two 64 x 17 outer-product blocks
+    ldk = lambda d: (d + 15) // 16 * 16 + 4  # noqa: E731
+    total = 4 * 16 * ((10 + 6 * 87) + 6 * 87 + (6 * ldk(87) + ldk(features)) + (ldk(10) + 5 * ldk(87))) + 2 * 64 * 17 * 4
+    assert (total <= 160 * 1024 - 1440) == (want == nat.PATH_NARROW)
+    assert lib.ipc_plan_create(ctypes.byref(h), 7, dims, 11, 0, 0, 1, 5, 1e-4, 0.5, 1, 0, -1) == nat.IPC_OK
+    try:
+        assert lib.ipc_plan_path(h) == want
+    finally:
+        lib.ipc_plan_destroy(h)
