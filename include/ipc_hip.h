@@ -60,6 +60,12 @@ extern "C" {
 #define IPC_ACT_GELU 5
 
 /* tile configurations of the MFMA GEMM family; IPC_TILE_AUTO picks by shape.
+ * The generic ids 0-2 name a small, a middle and a large output tile.  With
+ * fp32 storage they run on the k-chunk kernel (16 x 16, 32 x 32, 64 x 64
+ * tiles, the contraction split over a workgroup's waves; the automatic tile
+ * where that is larger) wherever that is the faster one, else on the tile kernel (32 x 32, 64 x 64, 128 x 128); the bits
+ * depend on the kernel, not on the tile.  With 16-bit storage the ids name the
+ * tile kernel, whose k order is the LDS-DMA kernel's.
  * IPC_TILE_DMA_* are the LDS-DMA kernel (operands streamed HBM -> LDS without
  * VGPR staging, transposed operands read with the LDS transpose read) in
  * four tile configurations: 256 x 128, 128 x 256,
@@ -71,7 +77,9 @@ extern "C" {
  * tensors and, for operands read transposed, a contiguous extent that is a
  * multiple of 8; IPC_TILE_AUTO picks the 256 x 256 one whenever those hold
  * and its tiles fill every CU at least once (256 tiles or more over the
- * groups), the 256 x 128 one when they hold otherwise; asking for a DMA tile
+ * groups), the 256 x 128 one when they hold otherwise, and the k-chunk kernel
+ * for calls of up to 256 tiles of 64 x 64 (inference update: 512), which use
+ * no workspace; asking for a DMA tile
  * where they do not hold is IPC_ERR_CONFIG.  The autotuner
  * searches all of them per shape. */
 #define IPC_TILE_AUTO (-1)

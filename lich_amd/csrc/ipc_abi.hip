@@ -107,15 +107,61 @@ int vec_ok(const void* p, long long contiguous, int esize) {
   return (contiguous % 4 == 0) && (reinterpret_cast<uintptr_t>(p) % (4 * esize) == 0);
 }
 
-// Auto tile: the largest tile that still yields at least ~2 workgroups per CU
-// (256 CUs), falling back to smaller tiles for the latency-bound shapes.
-int pick_tile(long long M, long long N, long long groups) {
-  const long long t128 = ((M + 127) / 128) * ((N + 127) / 128) * groups;
-  const long long t64 = ((M + 63) / 64) * ((N + 63) / 64) * groups;
-  if (t128 >= 512) return IPC_TILE_128x128;
-  if (t64 >= 256) return IPC_TILE_64x64;
-  if (M >= 64 && N >= 64 && t64 >= 64) return IPC_TILE_64x64;
-  return IPC_TILE_32x32;
+// Whether the k-chunk kernel (ipc_chunk_kernel.h) can address a problem: it
+// reads its operands through buffer resources, whose byte offsets, the rows of
+// a last, partly empty tile included, must stay below 2^31.
+bool chunk_fits(const GemmProblem& q, int esize) {
+  const long long a_rows = q.kind == KIND_INFER ? q.K : q.M, b_rows = q.kind == KIND_WEIGHT ? q.N : q.K;
+  return ((a_rows + 64) * q.lda + 64) * esize < (1LL << 31) && ((b_rows + 64) * q.ldb + 64) * esize < (1LL << 31);
+}
+
+// Output tiles of edge `e` over `n` problems.
+long long count_tiles(const GemmProblem* q, int n, int e) {
+  long long t = 0;
+  for (int i = 0; i < n; ++i) t += ((q[i].M + e - 1LL) / e) * ((q[i].N + e - 1LL) / e) * q[i].groups;
+  return t;
+}
+
+// Whether a launch over `n` problems that the LDS-DMA kernel does not run goes
+// to the k-chunk kernel: wherever that can address the operands, but for
+// * large fp32-storage predictions and weight updates, whose operands the tile
+//   kernel reads, and f(X) evaluates, half as often on its 128 x 128 tiles
+//   (MI355X, us, tile / k-chunk kernel, 4096 x 4096 x 2048 bf16 tanh:
+//   prediction split 2 517 / 565, weight update 468 / 559; inference 613 / 260);
+// * many tiles of few chunks, of which only as many of a workgroup's waves have
+//   work (prediction 2048 x 100 x 2048 20.8 / 39, split 2 2048 x 384 x 2048 43 /
+//   54; inference 4096 x 64 x 2048 29.7 / 54.8, 2048 x 256 x 2048 32 / 35.6,
+//   2048 x 384 x 2048 41.6 / 37.5; at 256 tiles of 64 x 64 the k-chunk kernel is
+//   ahead even at one chunk, inference 1024 x 100 x 1024 12.0 / 8.6, at 512 from
+//   two on, 2048 x 200 x 1024 20.9 / 17.3).
+bool use_chunk(const GemmProblem* q, int n, int esize) {
+  int kmax = 0;
+  for (int i = 0; i < n; ++i) {
+    if (!chunk_fits(q[i], esize)) return false;
+    kmax = std::max(kmax, q[i].K);
+  }
+  if (n == 0) return true;
+  const bool infer = q[0].kind == KIND_INFER;
+  const long long t64 = count_tiles(q, n, 64);
+  if (t64 > 256 && kmax <= 128) return false;
+  if (t64 > 512 && kmax <= (infer ? 256 : 512)) return false;
+  return !(esize == 4 && !infer && kmax >= 1024 && count_tiles(q, n, 128) >= 512);
+}
+
+// Tile of such a launch.  `tile`: IPC_TILE_AUTO, or a generic tile id, which
+// names the small, middle or large tile of either kernel, in the k-chunk kernel
+// the automatic one where that is larger (neither kernel's bits depend on the
+// tile).  Automatic: the largest tile that gives the 256
+// CUs about a workgroup each; a larger tile reads its operands less often, a
+// smaller one starts more waves.  MI355X, k-chunk kernel, fp32 storage, 16-bit
+// operands, us for 16 / 32 / 64: 512 x 512 x 2000 split 2 (256 large tiles)
+// 29.7 / 23.2 / 16.6, 512 x 784 x 256 (32 large, 128 middle tiles) 8.9 / 11.1
+// / 17.6, 1024^3 54 / 41 / 19.7.
+int pick_tile(int tile, const GemmProblem* q, int n, bool chunk) {
+  const long long t64 = count_tiles(q, n, 64);
+  if (chunk) return TILE_CHUNK_16 + std::max(tile, t64 >= 192 ? 2 : count_tiles(q, n, 32) >= 256 ? 1 : 0);
+  if (tile != IPC_TILE_AUTO) return tile;
+  return count_tiles(q, n, 128) >= 512 ? IPC_TILE_128x128 : t64 >= 64 ? IPC_TILE_64x64 : IPC_TILE_32x32;
 }
 
 int launch_rc(hipError_t err, const char* what) {
@@ -203,16 +249,27 @@ bool dma_eligible(int storage, int contraction, std::initializer_list<const void
   return true;
 }
 
-// Tile selection of a standalone call: returns 1 + the LDS-DMA configuration
+// Kernel selection of a standalone call: returns 1 + the LDS-DMA configuration
 // (0: 256 x 128, 1: 128 x 256, 2: 128 x 128, 3: 256 x 256) if that kernel runs it, 0 for
-// the generic kernel (tile resolved), or an error.
-int select_tile(int& tile, bool eligible, long long M, long long N, long long groups) {
+// the generic kernels, or an error.
+int select_tile(int tile, bool eligible, long long M, long long N, long long groups, bool infer = false) {
   const bool dma_tile = tile >= IPC_TILE_DMA_256x128;
   if (dma_tile && !eligible)
     return fail(IPC_ERR_CONFIG,
                 "tile %d (LDS-DMA) needs 16-bit storage, a contraction that is a multiple of %d, 16-byte "
                 "aligned tensors and row lengths that are multiples of 8", tile, WIDE_BK);
   if (eligible && tile == IPC_TILE_AUTO) {
+    // Few output tiles leave most CUs idle on 256 x 128 tiles; the k-chunk
+    // kernel then runs more and smaller ones and splits each one's
+    // contraction.  It wins up to 256 tiles of 64 x 64 (prediction and weight
+    // update), 512 for the inference update, whose operands both take the
+    // slower transposing reads here.  MI355X, bf16, us, LDS-DMA / k-chunk: at
+    // 256 tiles prediction 1024 x 4096 x 1024 relu 88 / 42, 1024^3 tanh 35 /
+    // 18, weight update 1024 x 1024, B = 512, relu 17.3 / 11.7; at 512
+    // prediction 4096 x 1024 x 512 relu 24 / 28, inference 2048 x 4096 x 1024
+    // tanh 89 / 65; at 1024 inference 4096 x 1024 x 1024 39 / 44.
+    const long long t64 = ((M + 63) / 64) * ((N + 63) / 64) * groups;
+    if (t64 <= (infer ? 512 : 256)) return 0;
     // 256 x 256 tiles (half the LDS reads per MFMA) once they fill every CU
     // (256) at least once, else 256 x 128: per-kernel sweep on MI355X, e.g.
     // M = K = 8192: prediction 0.26 -> 0.34, inference 0.31 -> 0.37, weight
@@ -222,8 +279,15 @@ int select_tile(int& tile, bool eligible, long long M, long long N, long long gr
     return t256 >= 256 ? 1 + IPC_TILE_DMA_256x256 - IPC_TILE_DMA_256x128 : 1;
   }
   if (dma_tile) return 1 + tile - IPC_TILE_DMA_256x128;
-  if (tile == IPC_TILE_AUTO) tile = pick_tile(M, N, groups);
   return 0;
+}
+
+// Tile of a standalone call that the LDS-DMA kernel does not run (`tile` as
+// asked for).  A generic tile asked for by id with 16-bit storage is the tile
+// kernel's, whose k order (and so every bit) is the LDS-DMA kernel's.
+int generic_tile(int tile, const GemmProblem& q, int storage) {
+  if (storage != IPC_DT_F32 && tile != IPC_TILE_AUTO) return tile;
+  return pick_tile(tile, &q, 1, use_chunk(&q, 1, elem_size(storage)));
 }
 
 // One WideProblem per group of a standalone 16-bit call.
@@ -386,8 +450,8 @@ int ipc_pred_err_ws(const void* x_upper, const void* w, const void* x_lower, voi
                    operand, act, use_dma - 1, workspace, workspace_bytes, stream, "ipc_pred_err");
   }
   GemmProblem p = make_pf(KIND_PRED, x_upper, w, x_lower, e, M, K, B, groups, act, es);
-  return launch_rc(launch_gemm(&p, 1, storage, operand, effective_split(storage, operand, split), tile,
-                               (hipStream_t)stream), "ipc_pred_err");
+  return launch_rc(launch_gemm(&p, 1, storage, operand, effective_split(storage, operand, split),
+                               generic_tile(tile, p, storage), (hipStream_t)stream), "ipc_pred_err");
 }
 
 int ipc_forward(const void* x_upper, const void* w, void* out, int M, int K, int B, int groups, int storage,
@@ -421,8 +485,8 @@ int ipc_forward_ws(const void* x_upper, const void* w, void* out, int M, int K, 
                    use_dma - 1, workspace, workspace_bytes, stream, "ipc_forward");
   }
   GemmProblem p = make_pf(KIND_FWD, x_upper, w, nullptr, out, M, K, B, groups, act, es);
-  return launch_rc(launch_gemm(&p, 1, storage, operand, effective_split(storage, operand, split), tile,
-                               (hipStream_t)stream), "ipc_forward");
+  return launch_rc(launch_gemm(&p, 1, storage, operand, effective_split(storage, operand, split),
+                               generic_tile(tile, p, storage), (hipStream_t)stream), "ipc_forward");
 }
 
 int ipc_infer_update(void* x, const void* e, const void* w_lower, const void* e_lower, void* a_out, int M,
@@ -446,7 +510,8 @@ int ipc_infer_update_ws(void* x, const void* e, const void* w_lower, const void*
   TRY(check_ptr(w_lower, "w_lower", es));
   TRY(check_ptr(e_lower, "e_lower", es));
   if (a_out) TRY(check_ptr(a_out, "a_out", es));
-  const int use_dma = select_tile(tile, dma_eligible(storage, K, {w_lower, e_lower}, {M, B}), M, B, groups);
+  const int use_dma = select_tile(tile, dma_eligible(storage, K, {w_lower, e_lower}, {M, B}), M, B, groups,
+                                  true);
   if (use_dma < 0) return use_dma;
   if (use_dma) {
     WideProblem q{};
@@ -462,7 +527,8 @@ int ipc_infer_update_ws(void* x, const void* e, const void* w_lower, const void*
                    "ipc_infer_update");
   }
   GemmProblem p = make_inf(x, e, w_lower, e_lower, a_out, M, K, B, groups, gamma, act, es);
-  return launch_rc(launch_gemm(&p, 1, storage, operand, IPC_SPLIT_NONE, tile, (hipStream_t)stream),
+  return launch_rc(launch_gemm(&p, 1, storage, operand, IPC_SPLIT_NONE, generic_tile(tile, p, storage),
+                               (hipStream_t)stream),
                    "ipc_infer_update");
 }
 
@@ -499,7 +565,8 @@ int ipc_weight_update_ws(void* w, const void* e, const void* x_upper, int M, int
                    "ipc_weight_update");
   }
   GemmProblem p = make_wgt(w, e, x_upper, M, K, B, groups, alpha, recompute, act, es);
-  return launch_rc(launch_gemm(&p, 1, storage, operand, IPC_SPLIT_NONE, tile, (hipStream_t)stream),
+  return launch_rc(launch_gemm(&p, 1, storage, operand, IPC_SPLIT_NONE, generic_tile(tile, p, storage),
+                               (hipStream_t)stream),
                    "ipc_weight_update");
 }
 
@@ -767,6 +834,21 @@ long long resident_eligible(int L, const int* dims, int B, int operand, int spli
   return resident_plan(dims, L, B, split == IPC_SPLIT_WX ? 3 : 1, 2, false, top_rows, ra);
 }
 
+// Kernels and tiles of the phased launches (tiles as set by ipc_plan_set_tiles
+// or automatic).  A net that the wide path could run as well keeps the tile
+// kernel: its k order is the wide path's, so the two paths' 16-bit operands
+// round alike and their states agree to fp32 rounding over many steps.
+void pick_phase_tiles(ipc_plan* plan) {
+  const bool chain = wide_eligible(plan->storage, plan->operand, plan->split, plan->wmode, plan->B);
+  const int es = elem_size(plan->storage), *t = plan->tile_override;
+  auto pick = [&](int want, const std::vector<GemmProblem>& v) {
+    return pick_tile(want, v.data(), (int)v.size(), !chain && use_chunk(v.data(), (int)v.size(), es));
+  };
+  plan->tile_pred = pick(t[0], plan->pred);
+  plan->tile_infer = pick(t[1], plan->infer);
+  plan->tile_weight = pick(t[2], plan->weight);
+}
+
 int launch_narrow_mode(ipc_plan* plan, int mode, int steps, hipStream_t s) {
   if (mode == NMODE_STEPS && plan->resident) {
     // The caches a resident launch keeps in the workspace (f(x[L]) images,
@@ -1009,17 +1091,8 @@ int ipc_plan_bind(ipc_plan* plan, void* const* x, void* const* e, void* const* w
   plan->act_dst = plan->recompute ? nullptr : a[L];
   for (int l = L - 1; l >= 1; --l)
     plan->fwd.push_back(make_pf(KIND_FWD, x[l + 1], w[l], nullptr, x[l], d[l], d[l + 1], B, 1, plan->act, es));
-  // One tile configuration per phase, chosen from the phase's total work.
-  long long rows_p = 0, rows_i = 0, rows_w = 0, cols_w = 0;
-  for (auto& q : plan->pred) rows_p += q.M;
-  for (auto& q : plan->infer) rows_i += q.M;
-  for (auto& q : plan->weight) { rows_w += q.M; cols_w = std::max(cols_w, (long long)q.N); }
-  plan->tile_pred = pick_tile(rows_p, B, 1);
-  plan->tile_infer = rows_i ? pick_tile(rows_i, B, 1) : 0;
-  plan->tile_weight = rows_w ? pick_tile(rows_w, cols_w, 1) : 0;
-  if (plan->tile_override[0] != IPC_TILE_AUTO) plan->tile_pred = plan->tile_override[0];
-  if (plan->tile_override[1] != IPC_TILE_AUTO) plan->tile_infer = plan->tile_override[1];
-  if (plan->tile_override[2] != IPC_TILE_AUTO) plan->tile_weight = plan->tile_override[2];
+  // One kernel and tile per phase (every layer of the phase is one launch).
+  pick_phase_tiles(plan);
   plan->launches = 1 + (plan->infer.empty() ? 0 : 1) + (plan->weight.empty() ? 0 : 1) + (int)plan->outer.size();
   if (plan->narrow) {
     TRY(bind_whole_step(plan->nargs, plan->resident ? &plan->rargs : nullptr, L, d.data(), B, x, e, w,
@@ -1241,7 +1314,9 @@ int ipc_plan_forward_init(ipc_plan* plan, void* stream) {
     return ok();
   }
   for (auto& q : plan->fwd) {
-    const int tile = pick_tile(q.M, q.N, 1);
+    // the prediction phase's kernel, so that its first hidden errors are
+    // exactly zero; the tile by this layer alone
+    const int tile = pick_tile(IPC_TILE_AUTO, &q, 1, plan->tile_pred >= TILE_CHUNK_16);
     TRY(launch_rc(launch_gemm(&q, 1, plan->storage, plan->operand, plan->split, tile, s), "plan forward init"));
   }
   return ok();
@@ -1264,11 +1339,7 @@ int ipc_plan_set_tiles(ipc_plan* plan, int tile_pred, int tile_infer, int tile_w
     if (t[i] != IPC_TILE_AUTO && (t[i] < IPC_TILE_32x32 || t[i] > IPC_TILE_128x128))
       return fail(IPC_ERR_CONFIG, "plan tile %d must be IPC_TILE_AUTO or a generic tile 0-2", t[i]);
   for (int i = 0; i < 3; ++i) plan->tile_override[i] = t[i];
-  if (plan->bound) {
-    if (t[0] != IPC_TILE_AUTO) plan->tile_pred = t[0];
-    if (t[1] != IPC_TILE_AUTO) plan->tile_infer = t[1];
-    if (t[2] != IPC_TILE_AUTO) plan->tile_weight = t[2];
-  }
+  if (plan->bound) pick_phase_tiles(plan);
   return ok();
 }
 

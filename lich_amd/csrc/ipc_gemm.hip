@@ -14,6 +14,14 @@ TileShape tile_shape(int tile) {
 hipError_t launch_gemm(const GemmProblem* probs, int count, int storage, int operand, int split, int tile,
                        hipStream_t s) {
   if (count <= 0) return hipSuccess;
+  if (tile >= TILE_CHUNK_16) {
+    switch (probs[0].kind) {
+      case KIND_PRED:
+      case KIND_FWD: return launch_chunk_pf(probs, count, storage, operand, split, tile, s);
+      case KIND_INFER: return launch_chunk_inf(probs, count, storage, operand, tile, s);
+      default: return launch_chunk_wgt(probs, count, storage, operand, tile, s);
+    }
+  }
   switch (probs[0].kind) {
     case KIND_PRED:
     case KIND_FWD: return launch_layout_pf(probs, count, storage, operand, split, tile, s);
