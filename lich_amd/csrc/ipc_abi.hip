@@ -614,7 +614,10 @@ struct ipc_plan {
   bool wdirect = false;  // wide, split 2: the prediction reads W itself (no Wh / Wl copies)
   std::vector<WideProblem> wpred, winfer, wweight, wfwd;  // wfwd: l = L-1 .. 1
   int pred_ksplit = 1;                                    // > 1: layer 0's prediction is k-split (last in wpred)
-  int wcfg[3] = {0, 0, 0};                                // tile configuration of the pred / infer / weight launches
+  int wcfg[3] = {-1, -1, -1};                             // tile configurations of the pred / infer / weight
+                                                          // launches as asked for (-1 = automatic) ...
+  int wrun[3] = {0, 0, 0};                                // ... and as they run
+  std::vector<int> wfwd_cfg;                              // those of the forward initialisation's launches
   int ksplit_request = 0;                                 // > 0: layer 0's k-split as set by the caller (1 = none)
   WideReduce wreduce{};                                   // its epilogue
   std::vector<WideCopy> wsync, wsync_init;               // wsync_init: W and x[L] only
@@ -1102,7 +1105,9 @@ int ipc_plan_bind(ipc_plan* plan, void* const* x, void* const* e, void* const* w
     plan->launches = 1;
   }
   if (plan->wide) {
-    const WideLayout lay(d, L, B, plan->split == IPC_SPLIT_W, plan->wcfg[0], plan->wdirect);
+    // the k-split (and so the bits) follows the configuration asked for, default 0
+    const int pred_cfg = std::max(plan->wcfg[0], 0);
+    const WideLayout lay(d, L, B, plan->split == IPC_SPLIT_W, pred_cfg, plan->wdirect);
     if (plan->wdirect)
       for (int l = 0; l < L; ++l)
         if (reinterpret_cast<uintptr_t>(w[l]) % 16 != 0)
@@ -1129,7 +1134,7 @@ int ipc_plan_bind(ipc_plan* plan, void* const* x, void* const* e, void* const* w
     if (hipGetDevice(&dev) != hipSuccess ||
         hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || ncu <= 0)
       ncu = 256;
-    plan->pred_ksplit = wide_pred_ksplit(d, L, B, plan->split == IPC_SPLIT_W, plan->wcfg[0], lay, ncu);
+    plan->pred_ksplit = wide_pred_ksplit(d, L, B, plan->split == IPC_SPLIT_W, pred_cfg, lay, ncu);
     if (plan->ksplit_request > 0) {
       const int k = plan->ksplit_request;
       if (k > lay.part_smax || (k > 1 && lay.wh[0].ld % ((long long)k * WIDE_BK) != 0))
@@ -1214,6 +1219,16 @@ int ipc_plan_bind(ipc_plan* plan, void* const* x, void* const* e, void* const* w
       q.vec = B % 4 == 0 && a16(x[l]);
       plan->wfwd.push_back(q);
     }
+    auto run_cfg = [&](int asked, int mode, const std::vector<WideProblem>& v) {
+      return asked >= 0 ? asked : wide_auto_config(mode, plan->split == IPC_SPLIT_W ? 2 : 1, v.data(), (int)v.size(),
+                                                  ncu);
+    };
+    plan->wrun[0] = run_cfg(plan->wcfg[0], WIDE_PRED, plan->wpred);
+    plan->wrun[1] = run_cfg(plan->wcfg[1], WIDE_INFER, plan->winfer);
+    plan->wrun[2] = run_cfg(plan->wcfg[2], WIDE_WEIGHT, plan->wweight);
+    plan->wfwd_cfg.clear();
+    for (auto& q : plan->wfwd)
+      plan->wfwd_cfg.push_back(wide_auto_config(WIDE_FWD, plan->split == IPC_SPLIT_W ? 2 : 1, &q, 1, ncu));
     TRY(launch_rc(wide_prepare(), "wide path LDS limit"));
     auto chunks = [](int n) { return (n + WIDE_MAX_BATCH - 1) / WIDE_MAX_BATCH; };
     plan->launches = 2 * chunks(L) + chunks(L - 1) + (plan->pred_ksplit > 1 ? 1 : 0);
@@ -1233,17 +1248,17 @@ int run_phase(ipc_plan* plan, int phase, hipStream_t s) {
     switch (phase) {
       case IPC_PHASE_PRED:
         TRY(launch_rc(launch_wide(WIDE_PRED, plan->wpred.data(), (int)plan->wpred.size(), plan->operand,
-                                  plan->split == IPC_SPLIT_W ? 2 : 1, plan->act, s, plan->wcfg[0], plan->wdirect),
+                                  plan->split == IPC_SPLIT_W ? 2 : 1, plan->act, s, plan->wrun[0], plan->wdirect),
                       "wide prediction phase"));
         if (plan->pred_ksplit > 1)
           return launch_rc(launch_wide_reduce(plan->wreduce, plan->operand, s), "wide prediction reduce");
         return ok();
       case IPC_PHASE_INFER:
         return launch_rc(launch_wide(WIDE_INFER, plan->winfer.data(), (int)plan->winfer.size(), plan->operand, 1,
-                                     plan->act, s, plan->wcfg[1]), "wide inference phase");
+                                     plan->act, s, plan->wrun[1]), "wide inference phase");
       default:
         return launch_rc(launch_wide(WIDE_WEIGHT, plan->wweight.data(), (int)plan->wweight.size(), plan->operand, 1,
-                                     plan->act, s, plan->wcfg[2]), "wide weight phase");
+                                     plan->act, s, plan->wrun[2]), "wide weight phase");
     }
   }
   switch (phase) {
@@ -1307,9 +1322,9 @@ int ipc_plan_forward_init(ipc_plan* plan, void* stream) {
     // kernel (its epilogue writes x[l] and the f(x[l]) copies the next layer reads)
     TRY(launch_rc(launch_wide_copy(plan->wsync_init.data(), (int)plan->wsync_init.size(), plan->operand, s),
                   "wide operand copies"));
-    for (auto& q : plan->wfwd)
-      TRY(launch_rc(launch_wide(WIDE_FWD, &q, 1, plan->operand, plan->split == IPC_SPLIT_W ? 2 : 1, plan->act, s, 0,
-                                plan->wdirect),
+    for (size_t i = 0; i < plan->wfwd.size(); ++i)
+      TRY(launch_rc(launch_wide(WIDE_FWD, &plan->wfwd[i], 1, plan->operand, plan->split == IPC_SPLIT_W ? 2 : 1,
+                                plan->act, s, plan->wfwd_cfg[i], plan->wdirect),
                     "wide forward init"));
     return ok();
   }
@@ -1365,11 +1380,11 @@ int ipc_plan_set_wide_config(ipc_plan* plan, int pred_cfg, int infer_cfg, int we
   }
   if (ksplit < -1 || ksplit == 0 || ksplit > 16 || (ksplit > 0 && (ksplit & (ksplit - 1))))
     return fail(IPC_ERR_CONFIG, "k-split must be -1 (automatic) or a power of two in [1, 16]; got %d", ksplit);
-  for (int ph = 0; ph < 3; ++ph) plan->wcfg[ph] = c[ph] < 0 ? 0 : c[ph];
+  for (int ph = 0; ph < 3; ++ph) plan->wcfg[ph] = c[ph];
   plan->ksplit_request = ksplit < 0 ? 0 : ksplit;
   // the prediction tile sets how many k-split slices the workspace holds
   plan->ws_bytes =
-      WideLayout(plan->dims, plan->L, plan->B, plan->split == IPC_SPLIT_W, plan->wcfg[0], plan->wdirect).total;
+      WideLayout(plan->dims, plan->L, plan->B, plan->split == IPC_SPLIT_W, std::max(plan->wcfg[0], 0), plan->wdirect).total;
   return ok();
 }
 

@@ -242,7 +242,7 @@ __global__ void __launch_bounds__(WGM * WGN * 64) dma_gemm_kernel(const Batch bt
   typedef typename MF::operand V;
   static_assert(S >= 2 && IA * 1024 * NW == A_BYTES && IB * 1024 * NW == B_BYTES && RB * 16 * NT == B_BYTES,
                 "tile / wave count");
-  static_assert(WTM % 32 == 0 && WTN % 32 == 0 && BM % 128 == 0 && BN % 128 == 0, "tile");
+  static_assert(WTM % 32 == 0 && WTN % 32 == 0 && BM % 64 == 0 && BN % 64 == 0, "tile");
   static_assert(!BREG || S16, "register-path operands belong to the standalone kernels");
 
   // XCD-aware renumbering: workgroup b runs on XCD b % 8; give every XCD a

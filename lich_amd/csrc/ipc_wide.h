@@ -101,9 +101,16 @@ struct WideReduce {
 };
 hipError_t launch_wide_reduce(const WideReduce& r, int operand, hipStream_t s);
 
+// Configuration index of the 64 x 64 tiles, which the plan picks for launches
+// with few default tiles (not one of the configurations a caller selects).
+constexpr int WIDE_CFG_SMALL = 100;
+
 // Tile configurations a phase offers (WIDE_PRED with split 1 or 2,
 // WIDE_INFER, WIDE_WEIGHT; 1 for WIDE_FWD); configuration 0 is the default.
 int wide_config_count(int mode, int split);
+
+// Configuration a launch over `count` problems runs by default on `ncu` CUs.
+int wide_auto_config(int mode, int split, const WideProblem* probs, int count, int ncu);
 
 // Output tile of prediction configuration `cfg` for `split` (1 or 2).
 void wide_pred_tile(int split, int cfg, int* bm, int* bn);

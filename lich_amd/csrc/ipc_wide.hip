@@ -2,6 +2,8 @@
 // over all layers of the LDS-DMA MFMA kernel of ipc_dma_gemm.h with the fused
 // epilogues that keep the fp32 masters and their 16-bit operand copies in
 // step, plus the kernel that re-derives the copies from the masters.
+#include <cmath>
+
 #include "ipc_dma_gemm.h"
 
 namespace ipc {
@@ -51,6 +53,14 @@ constexpr bool same_tiles() {
 static_assert(sizeof(kPred2ATiles) == sizeof(kPred2Tiles) && same_tiles(),
               "one a32 configuration, of the same tile, per split-2 prediction one");
 
+// Small tiles (64 x 64, 4 waves of 32 x 32) for launches whose default tiles
+// would leave most CUs idle (WIDE_CFG_SMALL; the plan picks it).  3 stages, 48
+// KB of LDS (72 with the split-2 prediction's fp32 or lo operand), so that a CU
+// holds three (two) workgroups: against 4 stages the same at one workgroup per
+// CU and faster beyond ((100, 1024 x 3, 784), B = 1024: prediction 45.0 -> 31.9
+// us, inference 26.9 -> 22.7, weight update 23.3 -> 20.0).
+#define WIDE_SMALL_CFG(X) X(64, 64, 3, 2, 2)
+
 // forward initialisation: the split-1 prediction tiles; split 2 keeps 128 x 128
 // (one layer per launch: its tiles fill all CUs once per 4096-row layer, 82 us
 // per layer against 120 us on the prediction's 128 x 256 tiles; the sums per
@@ -68,6 +78,9 @@ template <typename OT, int ACT, bool A32> using FwdCfg2 = Cfg<OT, WIDE_FWD, 2, A
 #define IPC_P2A(BM_, BN_, S_, WM_, WN_) IPC_CFG_CASE(WIDE_PRED, 2, ACT_IDENTITY, true, BM_, BN_, S_, WM_, WN_)
 #define IPC_IN(BM_, BN_, S_, WM_, WN_) IPC_CFG_CASE(WIDE_INFER, 1, ACT, false, BM_, BN_, S_, WM_, WN_)
 #define IPC_WT(BM_, BN_, S_, WM_, WN_) IPC_CFG_CASE(WIDE_WEIGHT, 1, ACT_IDENTITY, false, BM_, BN_, S_, WM_, WN_)
+#define IPC_F1(BM_, BN_, S_, WM_, WN_) IPC_CFG_CASE(WIDE_FWD, 1, ACT, false, BM_, BN_, S_, WM_, WN_)
+#define IPC_F2(BM_, BN_, S_, WM_, WN_) IPC_CFG_CASE(WIDE_FWD, 2, ACT, false, BM_, BN_, S_, WM_, WN_)
+#define IPC_F2A(BM_, BN_, S_, WM_, WN_) IPC_CFG_CASE(WIDE_FWD, 2, ACT, true, BM_, BN_, S_, WM_, WN_)
 
 template <typename OT>
 struct Phase {
@@ -78,6 +91,22 @@ struct Phase {
     static hipError_t run(int mode, int split, int cfg, bool prep, const WideProblem* probs, int count,
                           hipStream_t s, bool a32) {
       int i = 0;
+      if (cfg == WIDE_CFG_SMALL) {
+        cfg = 0;
+        switch (mode) {
+          case WIDE_PRED:
+            if (split == 2 && a32) { WIDE_SMALL_CFG(IPC_P2A) }
+            if (split == 2) { WIDE_SMALL_CFG(IPC_P2) }
+            WIDE_SMALL_CFG(IPC_P1)
+          case WIDE_INFER: WIDE_SMALL_CFG(IPC_IN)
+          case WIDE_WEIGHT: WIDE_SMALL_CFG(IPC_WT)
+          default:
+            if (split == 2 && a32) { WIDE_SMALL_CFG(IPC_F2A) }
+            if (split == 2) { WIDE_SMALL_CFG(IPC_F2) }
+            WIDE_SMALL_CFG(IPC_F1)
+        }
+        return hipErrorInvalidValue;
+      }
       switch (mode) {
         case WIDE_PRED:
           if (split == 2 && a32) { WIDE_PRED2A_CFGS(IPC_P2A) }
@@ -96,13 +125,21 @@ struct Phase {
   static hipError_t prepare() {
     hipError_t e;
     for (int act = 0; act < 6; ++act) {
+      if ((e = dma::by_act<Run>(act, WIDE_INFER, 1, WIDE_CFG_SMALL, true, nullptr, 0, nullptr, false)) != hipSuccess)
+        return e;
       for (int c = 0; c < kInferCfgs; ++c)
         if ((e = dma::by_act<Run>(act, WIDE_INFER, 1, c, true, nullptr, 0, nullptr, false)) != hipSuccess) return e;
       for (int sp = 1; sp <= 2; ++sp)
         for (int a32 = 0; a32 <= (sp == 2 ? 1 : 0); ++a32)
-          if ((e = dma::by_act<Run>(act, WIDE_FWD, sp, 0, true, nullptr, 0, nullptr, a32 != 0)) != hipSuccess)
-            return e;
+          for (int c : {0, WIDE_CFG_SMALL})
+            if ((e = dma::by_act<Run>(act, WIDE_FWD, sp, c, true, nullptr, 0, nullptr, a32 != 0)) != hipSuccess)
+              return e;
     }
+    for (int sp = 1; sp <= 2; ++sp)
+      for (int a32 = 0; a32 <= (sp == 2 ? 1 : 0); ++a32)
+        if ((e = Run<0>::run(WIDE_PRED, sp, WIDE_CFG_SMALL, true, nullptr, 0, nullptr, a32 != 0)) != hipSuccess)
+          return e;
+    if ((e = Run<0>::run(WIDE_WEIGHT, 1, WIDE_CFG_SMALL, true, nullptr, 0, nullptr, false)) != hipSuccess) return e;
     for (int c = 0; c < kPred1Cfgs; ++c)
       if ((e = Run<0>::run(WIDE_PRED, 1, c, true, nullptr, 0, nullptr, false)) != hipSuccess) return e;
     for (int c = 0; c < kPred2Cfgs; ++c)
@@ -289,7 +326,7 @@ hipError_t wide_prepare() {
 
 hipError_t launch_wide(int mode, const WideProblem* probs, int count, int operand, int split, int act,
                        hipStream_t s, int cfg, bool a32) {
-  if (cfg < 0 || cfg >= wide_config_count(mode, split)) return hipErrorInvalidValue;
+  if (cfg != WIDE_CFG_SMALL && (cfg < 0 || cfg >= wide_config_count(mode, split))) return hipErrorInvalidValue;
   if (a32 && (split != 2 || (mode != WIDE_PRED && mode != WIDE_FWD))) return hipErrorInvalidValue;
   for (int base = 0; base < count; base += WIDE_MAX_BATCH) {
     const int n = count - base < WIDE_MAX_BATCH ? count - base : WIDE_MAX_BATCH;
@@ -325,6 +362,52 @@ int wide_config_count(int mode, int split) {
     case WIDE_WEIGHT: return kWeightCfgs;
     default: return 1;
   }
+}
+
+// The configuration with the shortest estimated launch: `round` us of
+// prologue and epilogue plus `step` us per k-step of 64 for every round of
+// tiles over the device (`per_cu` workgroups of a configuration share a CU).
+// The constants are measured launches of nets of width 200-4096 at batch
+// 1-1024 (MI355X, us, default / best of these: (10, 512 x 3, 784), B = 256
+// prediction 27.5 / 9.8 on 64 x 64, inference 44.7 / 10.4, weight update 28.3 /
+// 8.2; (1000, 2048 x 4), B = 512 prediction 66.7 / 50.2 on 128 x 128, inference
+// 78.6 / 32.0 on 64 x 64, weight update 38.7 on the default; (1000, 4096 x 3),
+// B = 256 prediction 114 / 81, inference 120 / 34.9).  All give the same bits.
+int wide_auto_config(int mode, int split, const WideProblem* probs, int count, int ncu) {
+  struct Candidate { int cfg, bm, bn, per_cu; double round, step; };
+  static const Candidate pred1[] = {{0, 256, 128, 1, 6, 1.5}, {WIDE_CFG_SMALL, 64, 64, 2, 4, 0.5}};
+  static const Candidate pred2[] = {{0, 128, 256, 1, 4, 1.9}, {1, 128, 128, 1, 4, 1.3}, {WIDE_CFG_SMALL, 64, 64, 2, 3, 0.75}};
+  static const Candidate infer[] = {{0, 256, 256, 1, 34, 1.3}, {1, 128, 256, 1, 20, 0.85}, {WIDE_CFG_SMALL, 64, 64, 2, 4, 0.42}};
+  static const Candidate weight[] = {{0, 256, 256, 1, 30, 1.3}, {4, 128, 128, 1, 9.5, 0.75}, {WIDE_CFG_SMALL, 64, 64, 3, 5, 0.45}};
+  static const Candidate fwd1[] = {{0, 256, 128, 1, 6, 1.5}, {WIDE_CFG_SMALL, 64, 64, 2, 4, 0.5}};
+  static const Candidate fwd2[] = {{0, 128, 128, 1, 4, 1.3}, {WIDE_CFG_SMALL, 64, 64, 2, 3, 0.75}};
+  const Candidate* c = pred1;
+  int nc = 2;
+  switch (mode) {
+    case WIDE_PRED: if (split == 2) { c = pred2; nc = 3; } break;
+    case WIDE_INFER: c = infer; nc = 3; break;
+    case WIDE_WEIGHT: c = weight; nc = 3; break;
+    default: c = split == 2 ? fwd2 : fwd1; break;
+  }
+  int best = 0;
+  double best_t = 0.0;
+  for (int i = 0; i < nc; ++i) {
+    double tiles = 0.0, steps = 0.0, longest = 0.0;
+    for (int j = 0; j < count; ++j) {
+      const WideProblem& q = probs[j];
+      const double sl = q.ksplit > 1 ? q.ksplit : 1, ks = (double)(q.K / WIDE_BK) / sl;
+      const double t = sl * ((q.M + c[i].bm - 1) / c[i].bm) * ((q.N + c[i].bn - 1) / c[i].bn);
+      tiles += t;
+      steps += t * ks;
+      longest = ks > longest ? ks : longest;
+    }
+    if (tiles <= 0.0) return 0;
+    const double rounds = std::ceil(tiles / ((double)ncu * c[i].per_cu));
+    const double walk = rounds * steps / tiles;
+    const double t = rounds * c[i].round + c[i].step * (walk > longest ? walk : longest);
+    if (i == 0 || t < best_t) { best = c[i].cfg; best_t = t; }
+  }
+  return best;
 }
 
 #define IPC_TILE_XY(BM_, BN_, S_, WM_, WN_) if (cfg == i++) { *bm = BM_; *bn = BN_; return; }
