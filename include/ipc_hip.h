@@ -185,11 +185,12 @@ typedef struct ipc_plan ipc_plan;
 /* split applies to the prediction phase and the forward initialisation.
  * path selects the kernels a plan runs:
  *   IPC_PATH_AUTO    the layer-resident whole-step kernel when eligible (see
- *                    IPC_PATH_RESIDENT), else the column-block whole-step
- *                    kernel when the net is narrow (fp32 storage, every output
- *                    width d_0..d_{L-1} <= 128, L <= 16, split 1 or 3, one
- *                    column block's buffers fit in LDS), else the wide GEMM
- *                    path when eligible, else the phased path;
+ *                    IPC_PATH_RESIDENT); else, when the net is narrow (fp32
+ *                    storage, every output width d_0..d_{L-1} <= 128, L <= 16,
+ *                    split 1 or 3, one column block's buffers fit in LDS), the
+ *                    column-block whole-step kernel for widths <= 64 and B <=
+ *                    128 and the phased path beyond; else the wide GEMM path
+ *                    when eligible, else the phased path;
  *   IPC_PATH_PHASED  one generic multi-layer launch per phase (any config);
  *   IPC_PATH_NARROW  the column-block whole-step kernel (IPC_ERR_CONFIG if
  *                    not narrow);
@@ -371,9 +372,10 @@ int ipc_plan_graph_steps(const ipc_plan* plan);
  * No counterpart in the reference: an entry point for callers that cannot
  * allocate device memory (code under hipGraph capture, tight serving loops,
  * harnesses that forbid hipMalloc).  Runs `steps` iPC steps of a narrow net
- * on the whole-step kernels exactly as a plan created with IPC_PATH_AUTO,
- * fp32 storage and recompute mode would (ipc_plan_create + ipc_plan_bind +
- * ipc_plan_step: same kernels, same results), without a plan or a caller
+ * on the whole-step kernels exactly as a plan created with IPC_PATH_AUTO
+ * (widths above 64 or B above 128: IPC_PATH_NARROW), fp32 storage and
+ * recompute mode would (ipc_plan_create + ipc_plan_bind + ipc_plan_step: same
+ * kernels, same results), without a plan or a caller
  * workspace: the kernels' barrier words, f(x) buffers and exchange records
  * live in the library's static device scratch, 8 MiB per GPU, held until the
  * process ends.  A net that needs more is refused with IPC_ERR_SHAPE; one the

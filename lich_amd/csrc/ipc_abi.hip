@@ -824,6 +824,21 @@ bool narrow_outer(int B, int wmode) {
   return B <= NARROW_OUTER_MAX_B && (wmode == IPC_WMODE_OUTER || (wmode == IPC_WMODE_AUTO && B <= 16));
 }
 
+// Whether an automatic plan leaves a narrow net to the phased path's k-chunk
+// launches.  The column kernel's 16-column blocks re-read every W in a few
+// workgroups, phase after phase; the k-chunk kernel spreads the same products,
+// added in the same order, over the chip and is ahead at every measured size
+// (MI355X, us, initialisation / 4 steps, column kernel -> k-chunk launches:
+// 784 x 128^4 fp16 at B = 20, 128, 512, 1024 35 / 200 -> 21 / 72, 35 / 197 ->
+// 21 / 75, 35 / 247 -> 21 / 116, 36 / 349 -> 25 / 158; 784 x 128^2 fp32 at B =
+// 16 25 / 124 -> 14 / 68; 784 x 64^2 at B = 256 24 / 144 -> 17 / 75).  The
+// sizes the layer-resident kernel is laid out for (widths <= 64, B <= 128) keep
+// a whole-step kernel also where that one does not fit, so that a plan and
+// ipc_steps_noalloc, which only has those, agree there bit for bit.
+bool column_is_slow(int L, const int* dims, int B) {
+  return B > RES_MAX_B || *std::max_element(dims, dims + L) > RES_MAX_WIDTH;
+}
+
 // Layer-resident kernel eligibility; fills `ra` and returns its workspace bytes, or -1.
 // fp32 operands run it with either weight update (the rank-B one as the column
 // kernel computes it); 16-bit operands with the GEMM update only.
@@ -842,7 +857,8 @@ long long resident_eligible(int L, const int* dims, int B, int operand, int spli
 // kernel: its k order is the wide path's, so the two paths' 16-bit operands
 // round alike and their states agree to fp32 rounding over many steps.
 void pick_phase_tiles(ipc_plan* plan) {
-  const bool chain = wide_eligible(plan->storage, plan->operand, plan->split, plan->wmode, plan->B);
+  const bool chain = wide_eligible(plan->storage, plan->operand, plan->split, plan->wmode, plan->B) &&
+                     !narrow_eligible(plan->L, plan->dims.data(), plan->storage, plan->operand, plan->split);
   const int es = elem_size(plan->storage), *t = plan->tile_override;
   auto pick = [&](int want, const std::vector<GemmProblem>& v) {
     return pick_tile(want, v.data(), (int)v.size(), !chain && use_chunk(v.data(), (int)v.size(), es));
@@ -993,7 +1009,7 @@ int ipc_plan_create(ipc_plan** out, int L, const int* dims, int B, int storage, 
     }
   }
   int narrow_cap = 256;
-  if (eligible && (path == IPC_PATH_AUTO || path == IPC_PATH_NARROW || path == IPC_PATH_RESIDENT)) {
+  if (eligible && ((path == IPC_PATH_AUTO && !column_is_slow(L, dims, B)) || path == IPC_PATH_NARROW || path == IPC_PATH_RESIDENT)) {
     const int lds = narrow_lds_bytes(dims, L, operand, esplit);
     const int cap = coresident_capacity([&] { return narrow_prepare(operand, esplit, act, lds); },
                                         [&](int* n) { return narrow_occupancy(operand, esplit, act, lds, n); });
@@ -1018,8 +1034,9 @@ int ipc_plan_create(ipc_plan** out, int L, const int* dims, int B, int storage, 
   p->spin_limit = kNarrowSpinLimit;
   p->narrow_cap = narrow_cap;
   p->resident = path == IPC_PATH_RESIDENT || (path == IPC_PATH_AUTO && res_bytes >= 0);
-  p->narrow = p->resident || path == IPC_PATH_NARROW || (path == IPC_PATH_AUTO && eligible);
-  p->wide = !p->narrow && (path == IPC_PATH_WIDE || (path == IPC_PATH_AUTO && weligible));
+  const bool column = eligible && !column_is_slow(L, dims, B);
+  p->narrow = p->resident || path == IPC_PATH_NARROW || (path == IPC_PATH_AUTO && column);
+  p->wide = !p->narrow && (path == IPC_PATH_WIDE || (path == IPC_PATH_AUTO && weligible && !eligible));
   if (p->narrow) p->ws_bytes = narrow_workspace_bytes(dims, L, B, p->recompute != 0);
   if (p->resident) {
     p->rargs = ra;

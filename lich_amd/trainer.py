@@ -88,8 +88,9 @@ class IPCConfig:
     # policy file's tuned choice takes precedence.
     resident_rows: int | None = None
     # Kernel path: "auto" (the layer-resident whole-step kernel when eligible,
-    # else the column-block whole-step kernel for narrow nets, else the wide
-    # GEMM path when eligible, else phased), "resident", "narrow" / "on",
+    # else for narrow nets the column-block whole-step kernel up to width 64 and
+    # B = 128 and phased beyond, else the wide GEMM path when eligible, else
+    # phased), "resident", "narrow" / "on",
     # "wide", "phased" / "off".
     fused: str = "auto"
 

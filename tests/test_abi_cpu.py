@@ -650,18 +650,39 @@ def test_dma_tile_ids_are_refused_where_the_dma_kernel_cannot_run():
                                            (240, nat.PATH_PHASED)])
 def test_column_kernel_leaves_room_for_its_static_lds(features, want):
     """A column block whose buffers fill the LDS up to the kernel's static
-    1,440 bytes could not be launched (the LDS limit was refused): such a net
-    takes the phased path."""
+    1,440 bytes could not be launched (the LDS limit was refused): the column
+    kernel is refused for such a net, which takes the phased path (an automatic
+    plan does so at these widths in any case)."""
     lib = nat.lib()
     dims = (ctypes.c_int * 8)(10, 87, 87, 87, 87, 87, 87, features)
-    h = ctypes.c_void_p()
     # layout restated: raw x, eps, f(x) and eps operands of 16 columns (fp32: rows of
     # 16-padded contractions plus 4), two 64 x 17 outer-product blocks
     ldk = lambda d: (d + 15) // 16 * 16 + 4  # noqa: E731
     total = 4 * 16 * ((10 + 6 * 87) + 6 * 87 + (6 * ldk(87) + ldk(features)) + (ldk(10) + 5 * ldk(87))) + 2 * 64 * 17 * 4
     assert (total <= 160 * 1024 - 1440) == (want == nat.PATH_NARROW)
-    assert lib.ipc_plan_create(ctypes.byref(h), 7, dims, 11, 0, 0, 1, 5, 1e-4, 0.5, 1, 0, -1) == nat.IPC_OK
+    for path, got in ((nat.FUSED["narrow"], want), (nat.FUSED["auto"], nat.PATH_PHASED)):
+        h = ctypes.c_void_p()
+        rc = lib.ipc_plan_create(ctypes.byref(h), 7, dims, 11, 0, 0, 1, 5, 1e-4, 0.5, 1, 0, path)
+        if path == nat.FUSED["narrow"] and want != nat.PATH_NARROW:
+            assert rc == nat.ERR_CONFIG
+            continue
+        assert rc == nat.IPC_OK
+        try:
+            assert lib.ipc_plan_path(h) == got
+        finally:
+            lib.ipc_plan_destroy(h)
+
+
+@pytest.mark.parametrize("width,B,wmode,op,want", [
+    (64, 128, "gemm", "fp16", "resident"), (64, 129, "gemm", "fp16", "phased"), (65, 128, "gemm", "fp16", "phased"),
+    (64, 128, "gemm", "fp32", "narrow"), (64, 129, "gemm", "fp32", "phased"), (64, 16, "auto", "fp16", "narrow"),
+    (128, 1, "auto", "fp32", "phased"), (129, 128, "gemm", "fp16", "wide")])
+def test_automatic_path_of_narrow_nets(width, B, wmode, op, want):
+    lib, h = nat.lib(), ctypes.c_void_p()
+    dims = (ctypes.c_int * 5)(10, width, width, width, 784)
+    assert lib.ipc_plan_create(ctypes.byref(h), 4, dims, B, 0, {"fp32": nat.DT_F32, "fp16": nat.DT_F16}[op], 1,
+                               nat.act_code("tanh"), 1e-4, 0.5, 1, nat.WMODE[wmode], nat.FUSED["auto"]) == nat.IPC_OK
     try:
-        assert lib.ipc_plan_path(h) == want
+        assert nat.PATH_NAMES[lib.ipc_plan_path(h)] == want
     finally:
         lib.ipc_plan_destroy(h)
