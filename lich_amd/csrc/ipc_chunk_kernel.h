@@ -25,6 +25,7 @@
 // lr * NV + t (16 lanes read 16 * NV consecutive values).
 #pragma once
 
+#include <algorithm>
 #include <type_traits>
 
 #include "ipc_device.h"
@@ -246,16 +247,19 @@ constexpr int min_waves(int TM, int TN, int MAXW) {
   return TM * TN / 256 < MAXW ? TM * TN / 256 : MAXW;
 }
 
-template <typename ST, typename OT, int LAYOUT, int SPLIT, int TM, int TN, int MAXW>
-__global__ void __launch_bounds__(MAXW * 64) chunk_kernel(const GemmBatch batch) {
+// NS: waves that share a chunk, each with TN / NS of the tile's columns, where
+// the contraction has fewer chunks than the workgroup waves; OCC: waves per SIMD
+// the registers leave room for, that is workgroups a CU holds (run_chunk8).
+template <typename ST, typename OT, int LAYOUT, int SPLIT, int TM, int TN, int MAXW, int NS, int OCC>
+__global__ void __launch_bounds__(MAXW * 64, OCC) chunk_kernel(const GemmBatch batch) {
   using MM = Mma<OT>;
   typedef typename MM::operand V;
-  constexpr int KS = MM::KS, KL = MM::KL, RM = TM / 16, RN = TN / 16;
+  constexpr int KS = MM::KS, KL = MM::KL, RM = TM / 16, RN = TN / 16 / NS;
   constexpr bool A_KMAJ = LAYOUT != LAYOUT_INF, B_KMAJ = LAYOUT == LAYOUT_WGT;
   constexpr bool SA = SPLIT >= 2, SB = SPLIT >= 3;
   constexpr int LDP = TN + 4;                       // floats per row of a partial tile
   constexpr int STEPS = CHUNK_K / KS;
-  extern __shared__ __align__(16) float part[];     // [waves][TM][LDP]
+  extern __shared__ __align__(16) float part[];     // [chunks in flight][TM][LDP]
 
   const int bid = blockIdx.x;
   int pi = 0;
@@ -279,7 +283,8 @@ __global__ void __launch_bounds__(MAXW * 64) chunk_kernel(const GemmBatch batch)
 
   const int tid = threadIdx.x, nthreads = blockDim.x, lane = tid & 63, lr = tid & 15, lg = lane >> 4;
   // (uniform, so that the chunk's addresses are scalar)
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), waves = nthreads >> 6;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), slots = (nthreads >> 6) / NS;
+  const int slot = wave / NS, nw = wave % NS * (TN / NS);  // this wave's chunk of a round, its first column
   const int chunks = (K + CHUNK_K - 1) / CHUNK_K;
 
   // The epilogue's 4-column groups: group tid, then every nthreads (at most
@@ -319,8 +324,8 @@ __global__ void __launch_bounds__(MAXW * 64) chunk_kernel(const GemmBatch batch)
     if (LAYOUT == LAYOUT_INF) load_group(aux, ldx, ve, gi, es[i]);
   }
 
-  for (int c0 = 0; c0 < chunks; c0 += waves) {
-    const int c = c0 + wave;
+  for (int c0 = 0; c0 < chunks; c0 += slots) {
+    const int c = c0 + slot;
     if (c < chunks) {
       f32x4 acc[RM][RN];
 #pragma unroll
@@ -333,7 +338,7 @@ __global__ void __launch_bounds__(MAXW * 64) chunk_kernel(const GemmBatch batch)
         // k-steps whose loads are issued together: as many as about half of
         // the registers hold
         constexpr int REGS = (RM + RN) * KL * (ODD ? 4 : (int)sizeof(ST)) / 4;
-        constexpr int ROOM = MAXW > 8 ? (ODD ? 16 : 48) : TM > 32 ? 96 : 128;
+        constexpr int ROOM = MAXW > 8 ? (ODD ? 16 : 48) : OCC >= 4 ? 48 : TM > 32 ? 96 : 128;
         constexpr int AHEAD = REGS * STEPS <= ROOM ? STEPS : REGS * STEPS <= 2 * ROOM ? STEPS / 2
                               : REGS * STEPS <= 4 * ROOM ? STEPS / 4 : 1;
         Raw<ST, RM, KL> ra[AHEAD];
@@ -346,8 +351,8 @@ __global__ void __launch_bounds__(MAXW * 64) chunk_kernel(const GemmBatch batch)
             const int k = k0 + s * KS + lg * KL;
             if constexpr (A_KMAJ) load_kmaj<ST, RM, KL, ODD>(A, lda, m0, k, K, tail, lr, ra[s]);
             else load_mn<ST, RM, KL, ODD>(A, lda, m0, k, K, lr, ra[s]);
-            if constexpr (B_KMAJ) load_kmaj<ST, RN, KL, ODD>(B, ldb, n0, k, K, tail, lr, rb[s]);
-            else load_mn<ST, RN, KL, ODD>(B, ldb, n0, k, K, lr, rb[s]);
+            if constexpr (B_KMAJ) load_kmaj<ST, RN, KL, ODD>(B, ldb, n0 + nw, k, K, tail, lr, rb[s]);
+            else load_mn<ST, RN, KL, ODD>(B, ldb, n0 + nw, k, K, lr, rb[s]);
           }
 #pragma unroll
           for (int s = 0; s < AHEAD; ++s) {
@@ -402,7 +407,7 @@ __global__ void __launch_bounds__(MAXW * 64) chunk_kernel(const GemmBatch batch)
       }
       // the partial tile in matrix order: result register q of tile (i, j) is
       // operand row 4 lg + q of row tile i, column lr of column tile j
-      float* pw = part + wave * TM * LDP;
+      float* pw = part + slot * TM * LDP + nw;
 #pragma unroll
       for (int i = 0; i < RM; ++i)
 #pragma unroll
@@ -418,16 +423,16 @@ __global__ void __launch_bounds__(MAXW * 64) chunk_kernel(const GemmBatch batch)
         }
     }
     __syncthreads();
-    const int have = chunks - c0 < waves ? chunks - c0 : waves;
-    const bool last = c0 + waves >= chunks;
+    const int have = chunks - c0 < slots ? chunks - c0 : slots;
+    const bool last = c0 + slots >= chunks;
 #pragma unroll
     for (int u = 0; u < PRE; ++u) {
       const int gi = tid + u * nthreads;
       if (gi >= GROUPS) break;
       const int r = gi / (TN / 4), cc = (gi % (TN / 4)) * 4;
       float* at = part + r * LDP + cc;
-      // running sum of the earlier rounds: kept after the waves' partial tiles
-      float* run = part + waves * TM * LDP + r * LDP + cc;
+      // running sum of the earlier rounds: kept after the chunks' partial tiles
+      float* run = part + slots * TM * LDP + r * LDP + cc;
       float4 t = *reinterpret_cast<float4*>(at);
       float s[4] = {t.x, t.y, t.z, t.w};
       if (c0 > 0) {
@@ -478,11 +483,11 @@ __global__ void __launch_bounds__(MAXW * 64) chunk_kernel(const GemmBatch batch)
 }
 
 // Launch of one tile size over a ragged batch.
-template <typename ST, typename OT, int LAYOUT, int SPLIT, int TM, int TN, int MAXW>
+template <typename ST, typename OT, int LAYOUT, int SPLIT, int TM, int TN, int MAXW, int NS, int OCC>
 static hipError_t run_chunk(const GemmProblem* probs, int count, hipStream_t s) {
-  const void* fn = reinterpret_cast<const void*>(&chunk_kernel<ST, OT, LAYOUT, SPLIT, TM, TN, MAXW>);
+  const void* fn = reinterpret_cast<const void*>(&chunk_kernel<ST, OT, LAYOUT, SPLIT, TM, TN, MAXW, NS, OCC>);
   constexpr int TILE_BYTES = TM * (TN + 4) * 4;
-  constexpr int LDS_MAX = (MAXW + 1) * TILE_BYTES;
+  constexpr int LDS_MAX = (MAXW / NS + 1) * TILE_BYTES;
   static_assert(LDS_MAX <= 160 * 1024, "partial tiles exceed the LDS");
   if (LDS_MAX > 64 * 1024) {
     static const hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, LDS_MAX);
@@ -491,32 +496,67 @@ static hipError_t run_chunk(const GemmProblem* probs, int count, hipStream_t s) 
   for (int base = 0; base < count; base += MAX_BATCH) {
     GemmBatch batch;
     batch.count = count - base < MAX_BATCH ? count - base : MAX_BATCH;
-    int total = 0, waves = min_waves(TM, TN, MAXW), rounds = 1;
+    int total = 0, most = 1;
     for (int i = 0; i < batch.count; ++i) {
       const GemmProblem& q = probs[base + i];
       batch.p[i] = q;
       batch.start[i] = total;
       total += ((q.N + TN - 1) / TN) * ((q.M + TM - 1) / TM) * q.groups;
-      const int chunks = (q.K + CHUNK_K - 1) / CHUNK_K;
-      waves = chunks > waves ? (chunks < MAXW ? chunks : MAXW) : waves;
-      rounds = chunks > MAXW ? 2 : rounds;
+      most = std::max(most, (q.K + CHUNK_K - 1) / CHUNK_K);
     }
     for (int i = batch.count; i <= MAX_BATCH; ++i) batch.start[i] = total;
     if (total == 0) continue;
+    // partial tiles: a round's chunks, and the running sum where there are more
+    // rounds; no more than that, so that a CU holds several workgroups of few
+    // chunks
+    const int slots = std::min(most, MAXW / NS), waves = std::max(min_waves(TM, TN, MAXW), slots * NS);
+    const int tiles = most > slots ? slots + 1 : slots;
     void* args[] = {&batch};
-    const hipError_t err = hipLaunchKernel(fn, dim3(total), dim3(waves * 64), args,
-                                           (size_t)(waves + (rounds > 1 ? 1 : 0)) * TILE_BYTES, s);
+    const hipError_t err = hipLaunchKernel(fn, dim3(total), dim3(waves * 64), args, (size_t)tiles * TILE_BYTES, s);
     if (err != hipSuccess) return err;
   }
   return hipSuccess;
 }
 
+// Waves per chunk: where the longest contraction leaves an 8-wave workgroup
+// without a chunk for every wave, 2 or 4 waves take columns of one chunk each.
+// An operand A is then read by all of them, so the inference update, whose
+// narrower transposing reads cost more (1000 x 200 x 1000 10.4 -> 12.9 us), and
+// 16-bit storage with two (2000 x 400 x 500 weight update 16.7 -> 24) keep one.
+// MI355X, us, one wave a chunk / this rule: weight update 1000 x 1531, B = 300,
+// fp32 storage, bf16 operands 29.7 / 20.1, fp32 operands 44.4 / 28.7, bf16
+// storage 32.5 / 21.6; 1024 x 1024, B = 128, 13.6 / 9.5, 21.1 / 10.3, 14.6 / 8.9;
+// prediction 1000 x 200 x 1000 12.0 / 9.4, 19.0 / 10.8, 12.5 / 9.1.
+//
+// Workgroups per CU: two of 32 x 32 tiles, each with fewer loads in flight,
+// hide one another's latencies and reductions (prediction 1000 x 1531 x 300,
+// the three types in the same order, 37.1 -> 27.0 us, 48.8 -> 33.4, 36.1 -> 28.0;
+// inference 800 x 800 x 400 17.5 -> 12.3, 26.8 -> 21.0, 14.7 -> 11.4); an inference
+// update of at most one tile per CU keeps the loads instead (512 x 4096 x 512,
+// fp32, 42.7 us against 54.7).
+template <typename ST, typename OT, int LAYOUT, int SPLIT, int TM, int TN>
+static hipError_t run_chunk8(const GemmProblem* probs, int count, hipStream_t s) {
+  constexpr bool wide = sizeof(ST) == 4;
+  int kmax = 0;
+  for (int i = 0; i < count; ++i) kmax = std::max(kmax, probs[i].K);
+  if constexpr (LAYOUT != LAYOUT_INF && TN == 64)
+    if (kmax <= (wide ? 2 : 3) * CHUNK_K) return run_chunk<ST, OT, LAYOUT, SPLIT, TM, TN, 8, 4, 4>(probs, count, s);
+  if constexpr (LAYOUT != LAYOUT_INF && (wide || (LAYOUT == LAYOUT_WGT && TN == 32)))
+    if (kmax <= 4 * CHUNK_K) return run_chunk<ST, OT, LAYOUT, SPLIT, TM, TN, 8, 2, 4>(probs, count, s);
+  if constexpr (TN == 32) {
+    long long tiles = 0;
+    for (int i = 0; i < count; ++i) tiles += ((probs[i].M + 31LL) / 32) * ((probs[i].N + 31LL) / 32) * probs[i].groups;
+    if (LAYOUT != LAYOUT_INF || tiles > 256) return run_chunk<ST, OT, LAYOUT, SPLIT, TM, TN, 8, 1, 4>(probs, count, s);
+  }
+  return run_chunk<ST, OT, LAYOUT, SPLIT, TM, TN, 8, 1, 2>(probs, count, s);
+}
+
 template <typename ST, typename OT, int LAYOUT, int SPLIT>
 static hipError_t run_chunks(const GemmProblem* probs, int count, int tile, hipStream_t s) {
   switch (tile) {
-    case TILE_CHUNK_16: return run_chunk<ST, OT, LAYOUT, SPLIT, 16, 16, 16>(probs, count, s);
-    case TILE_CHUNK_32: return run_chunk<ST, OT, LAYOUT, SPLIT, 32, 32, 8>(probs, count, s);
-    default: return run_chunk<ST, OT, LAYOUT, SPLIT, 64, 64, 8>(probs, count, s);
+    case TILE_CHUNK_16: return run_chunk<ST, OT, LAYOUT, SPLIT, 16, 16, 16, 1, 4>(probs, count, s);
+    case TILE_CHUNK_32: return run_chunk8<ST, OT, LAYOUT, SPLIT, 32, 32>(probs, count, s);
+    default: return run_chunk8<ST, OT, LAYOUT, SPLIT, 64, 64>(probs, count, s);
   }
 }
 
