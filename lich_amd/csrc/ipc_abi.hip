@@ -249,10 +249,23 @@ bool dma_eligible(int storage, int contraction, std::initializer_list<const void
   return true;
 }
 
+// LDS-DMA configuration of an automatic call without an activation to evaluate.
+int s16_auto_config(long long M, long long N, long long groups) {
+  // 256 x 256 tiles (half the LDS reads per MFMA) once they fill every CU
+  // (256) at least once, else 256 x 128: per-kernel sweep on MI355X, e.g.
+  // M = K = 8192: prediction 0.26 -> 0.34, inference 0.31 -> 0.37, weight
+  // update 0.40 -> 0.43 of the bf16 peak; at 128 tiles of 256 x 256 half the
+  // CUs idle and the smaller tile wins
+  const long long t256 = ((M + 255) / 256) * ((N + 255) / 256) * groups;
+  return t256 >= 256 ? IPC_TILE_DMA_256x256 - IPC_TILE_DMA_256x128 : 0;
+}
+
 // Kernel selection of a standalone call: returns 1 + the LDS-DMA configuration
-// (0: 256 x 128, 1: 128 x 256, 2: 128 x 128, 3: 256 x 256) if that kernel runs it, 0 for
-// the generic kernels, or an error.
-int select_tile(int tile, bool eligible, long long M, long long N, long long groups, bool infer = false) {
+// (0: 256 x 128, 1: 128 x 256, 2: 128 x 128, 3: 256 x 256, S16_CFG_TALL: 512 x 64) if
+// that kernel runs it, 0 for the generic kernels, or an error.
+// `loader_act`: the activation the kernel's loader evaluates (identity: none).
+int select_tile(int tile, bool eligible, long long M, long long N, long long groups, bool infer = false,
+                int loader_act = IPC_ACT_IDENTITY) {
   const bool dma_tile = tile >= IPC_TILE_DMA_256x128;
   if (dma_tile && !eligible)
     return fail(IPC_ERR_CONFIG,
@@ -270,13 +283,15 @@ int select_tile(int tile, bool eligible, long long M, long long N, long long gro
     // tanh 89 / 65; at 1024 inference 4096 x 1024 x 1024 39 / 44.
     const long long t64 = ((M + 63) / 64) * ((N + 63) / 64) * groups;
     if (t64 <= (infer ? 512 : 256)) return 0;
-    // 256 x 256 tiles (half the LDS reads per MFMA) once they fill every CU
-    // (256) at least once, else 256 x 128: per-kernel sweep on MI355X, e.g.
-    // M = K = 8192: prediction 0.26 -> 0.34, inference 0.31 -> 0.37, weight
-    // update 0.40 -> 0.43 of the bf16 peak; at 128 tiles of 256 x 256 half the
-    // CUs idle and the smaller tile wins
-    const long long t256 = ((M + 255) / 256) * ((N + 255) / 256) * groups;
-    return t256 >= 256 ? 1 + IPC_TILE_DMA_256x256 - IPC_TILE_DMA_256x128 : 1;
+    // The tall tiles where they pad no more rows than 256 x 128 ones
+    // (S16_CFG_TALL has the measurements); not for tanh, the cheapest of its
+    // activations, where the 256 x 256 tiles fill the CUs (us, 256 x 256 / tall:
+    // 8192^3 tanh 1993 / 2036, sigmoid 2454 / 2266; 4096 x 2048 x 4096 tanh 132 /
+    // 138, sigmoid 162 / 152).
+    const int cfg = s16_auto_config(M, N, groups);
+    const long long t128 = ((M + 255) / 256) * ((N + 127) / 128), tall = ((M + 511) / 512) * ((N + 63) / 64);
+    if (s16_costly(loader_act) && tall <= t128 && (cfg == 0 || loader_act != IPC_ACT_TANH)) return 1 + S16_CFG_TALL;
+    return 1 + cfg;
   }
   if (dma_tile) return 1 + tile - IPC_TILE_DMA_256x128;
   return 0;
@@ -352,6 +367,7 @@ int run_s16(int mode, const WideProblem& q, int groups, long long a_gs, long lon
   hipStream_t s = (hipStream_t)stream;
   const long long need = s16_workspace_need(mode, act, q.M, q.K, b_gs, groups);
   if (need > 0 && workspace && ws_bytes >= need) {
+    if (cfg == S16_CFG_TALL) cfg = s16_auto_config(q.M, q.N, groups);  // f(X) no longer in the loader
     WideProblem qa = q;
     if (mode == S16_INFER) {
       // W_lower [K][M] -> [M][K] and E_lower [K][B] -> [B][K] (identity
@@ -437,7 +453,7 @@ int ipc_pred_err_ws(const void* x_upper, const void* w, const void* x_lower, voi
   TRY(check_ptr(w, "w", es));
   TRY(check_ptr(x_lower, "x_lower", es));
   TRY(check_ptr(e, "e", es));
-  const int use_dma = select_tile(tile, dma_eligible(storage, K, {x_upper, w}, {K, B}), M, B, groups);
+  const int use_dma = select_tile(tile, dma_eligible(storage, K, {x_upper, w}, {K, B}), M, B, groups, false, act);
   if (use_dma < 0) return use_dma;
   if (use_dma) {
     WideProblem q{};
@@ -472,7 +488,7 @@ int ipc_forward_ws(const void* x_upper, const void* w, void* out, int M, int K, 
   TRY(check_ptr(x_upper, "x_upper", es));
   TRY(check_ptr(w, "w", es));
   TRY(check_ptr(out, "out", es));
-  const int use_dma = select_tile(tile, dma_eligible(storage, K, {x_upper, w}, {K, B}), M, B, groups);
+  const int use_dma = select_tile(tile, dma_eligible(storage, K, {x_upper, w}, {K, B}), M, B, groups, false, act);
   if (use_dma < 0) return use_dma;
   if (use_dma) {
     WideProblem q{};

@@ -14,7 +14,7 @@
 //     of row r stored at chunk c ^ ((r >> 1) & 7): a 16-byte fragment read by
 //     16 lanes of 16 consecutive rows touches each of the 64 LDS banks once;
 //   * an m/n-contiguous block is 64 k-rows of 2*EDGE bytes, chunk c of k-row
-//     r at chunk c ^ ((r & 3) << 2); its fragments come from two
+//     r at chunk c ^ ((r & 3) << 2) (64 wide: ((r >> 1) & 1) << 2); its fragments come from two
 //     ds_read_b64_tr_b16 (16 lanes read a 4 x 16 block, one 8-byte row piece
 //     each, and get its columns back), and the swizzle spreads the 4 k-rows of
 //     a half-wave over distinct banks;
@@ -87,7 +87,12 @@ constexpr bool s16_infer(int mode) { return mode == S16_INFER || mode == S16_INF
 
 // chunk position of chunk c in row r
 __device__ __forceinline__ int kc_swz(int r, int c) { return c ^ ((r >> 1) & 7); }
-__device__ __forceinline__ int mn_swz(int r, int c) { return c ^ ((r & 3) << 2); }
+// (64 columns: 8 chunks a row; rows r and r + 2 fall on the same banks)
+template <int EDGE>
+__device__ __forceinline__ int mn_swz(int r, int c) {
+  static_assert(EDGE >= 64, "two 32-wide blocks a row at least");
+  return c ^ ((EDGE == 64 ? (r >> 1) & 1 : r & 3) << 2);
+}
 
 // Global source of LDS slot `slot` (16 bytes) of an operand block.
 //   KC: rows e0 .. e0+EDGE-1 (clamped to lim-1), k0 .. k0+63
@@ -109,7 +114,7 @@ __device__ __forceinline__ const OT* slot_src(const OT* g, long long ld, int e0,
     return g + (long long)row * ld + k0 + c * 8;
   } else {
     constexpr int CPR = EDGE / 8;  // chunks per k-row
-    const int r = slot / CPR, c = mn_swz(r, slot % CPR);
+    const int r = slot / CPR, c = mn_swz<EDGE>(r, slot % CPR);
     const int col = e0 + c * 8 <= lim - 8 ? e0 + c * 8 : lim - 8;
     return g + (long long)(k0 + r) * ld + col;
   }
@@ -417,7 +422,7 @@ __global__ void __launch_bounds__(WGM * WGN * 64) dma_gemm_kernel(const Batch bt
   };
   auto frag_mn = [&](const unsigned char* blk, int rowb, int col0, int kk) -> V {
     // col0: first column of the 32-wide block (multiple of 32)
-    const int chunk = ((((col0 >> 5) ^ tr_x)) << 2) | tr_low;
+    const int chunk = (((col0 >> 5) ^ (rowb == 128 ? tr_x >> 1 : tr_x)) << 2) | tr_low;
     const unsigned char* p0 = blk + (kk * 16 + tr_row) * rowb + (chunk << 4) + tr_half;
     const s16x4 v0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(p0));
     const s16x4 v1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(p0 + 4 * rowb));

@@ -19,6 +19,36 @@ namespace {
 // 64 each), within +-3 % of 16.
 using Tiles0 = s16::Tiles<256, 128, 3, 4, 4, 4, 2>;
 
+// Tall tiles (S16_CFG_TALL): 512 x 64, 8 waves of 64 x 64, 2 stages, for the
+// prediction and forward whose loader evaluates an exponential activation.
+// The loader's VALU work bounds those, and a tile of twice the rows evaluates
+// f(X_upper) half as often.  MI355X, bf16, us, 256 x 128 / this: 4096 x 4096 x
+// 2048 tanh 135 / 126, sigmoid 164 / 145, gelu 154 / 138, silu 175 / 148; 8192 x
+// 2048 x 1000 75 / 73, 88 / 80, 84 / 78, 90 / 81 (relu 105 / 119, 56 / 65: stays).
+template <typename OT>
+struct Tall {
+  template <int ACT>
+  struct Run {
+    static hipError_t run(int mode, const WideProblem* probs, int count, hipStream_t s) {
+      if constexpr (s16_costly(ACT)) {
+        if (mode == S16_PRED) return dma::Cfg<OT, S16_PRED, 1, ACT, true, 512, 64, 2, 8, 1>::launch(probs, count, s);
+        if (mode == S16_FWD) return dma::Cfg<OT, S16_FWD, 1, ACT, true, 512, 64, 2, 8, 1>::launch(probs, count, s);
+      }
+      return hipErrorInvalidValue;
+    }
+  };
+};
+
+hipError_t launch_tall(int mode, const WideProblem* probs, int count, int operand, int act, hipStream_t s) {
+  for (int base = 0; base < count; base += WIDE_MAX_BATCH) {
+    const int n = std::min(count - base, WIDE_MAX_BATCH);
+    const hipError_t e = operand == DT_F16 ? dma::by_act<Tall<f16>::template Run>(act, mode, probs + base, n, s)
+                                           : dma::by_act<Tall<bf16>::template Run>(act, mode, probs + base, n, s);
+    if (e != hipSuccess) return e;
+  }
+  return hipSuccess;
+}
+
 // out[i] = f(in[i]) rounded to the storage type: the register path's value
 // (f in fp32 of the stored 16-bit input, then one rounding), 8 elements per
 // thread when the buffers allow 16-byte accesses.
@@ -164,6 +194,7 @@ hipError_t launch_s16(int mode, const WideProblem* probs, int count, int operand
     case 1: return s16::launch_tiles1(mode, probs, count, operand, act, s);
     case 2: return s16::launch_tiles2(mode, probs, count, operand, act, s);
     case 3: return s16::launch_tiles3(mode, probs, count, operand, act, s);
+    case S16_CFG_TALL: return launch_tall(mode, probs, count, operand, act, s);
     default: return hipErrorInvalidValue;
   }
 }

@@ -131,6 +131,11 @@ bool wide_problem_ok(int mode, int split, bool a32, const WideProblem& q);
 // Raises the dynamic-LDS limit of every wide-path kernel instantiation.
 hipError_t wide_prepare();
 
+// Internal configuration of launch_s16: 512 x 64 tiles for the prediction and
+// forward with an exponential activation in the loader (ipc_s16.hip).
+constexpr int S16_CFG_TALL = 4;
+constexpr bool s16_costly(int act) { return act >= 2; }  // tanh, sigmoid, silu, gelu
+
 // Standalone 16-bit-storage launches (modes S16_*) over `count` problems.
 // `act`: the loader activation of S16_PRED / S16_FWD / S16_WEIGHT (ACT_IDENTITY
 // for a saved activation), the epilogue activation of S16_INFER.
