@@ -12,7 +12,7 @@
 // rows, each lane 4 adjacent columns.  What bounds it is W in memory, so a
 // thread's loads of W (16 bytes each) are issued before anything else and
 // arrive while the rows X[k0 .. k0 + OUTER_TK) are activated, once per element,
-// into LDS as [B][OUTER_TK].  MI355X, fp32 2048 x 2048, B = 8: 7.7 us (4.4 TB/s
+// into LDS as [B][OUTER_TK].  MI355X, fp32 2048 x 2048, B = 8: 8.4 us (4.0 TB/s
 // of W), against 15.8 with W loaded after the sums, 4 bytes a lane; bf16 8192 x
 // 8192, B = 16: 79 us against 246.
 #include "ipc_device.h"
@@ -159,7 +159,7 @@ template <typename ST>
 static hipError_t run_outer_as(const OuterProblem& p, hipStream_t s) {
   const bool vec = p.K % 4 == 0 && reinterpret_cast<uintptr_t>(p.w) % (4 * sizeof(ST)) == 0;
   // 16 rows a workgroup once that gives every CU two of them, else 8 (MI355X,
-  // us, 8 / 16 / 32 rows: fp32 2048 x 2048, B = 8, 8.3 / 7.7 / 7.7; bf16 8192 x
+  // us, 8 / 16 / 32 rows: fp32 2048 x 2048, B = 8, 8.3 / 7.7 / 7.7 back to back; bf16 8192 x
   // 8192, B = 16, 116 / 79 / 68; fp16, B = 1, 47 / 41 / 44; bf16 1000 x 1531, B =
   // 5, 378 workgroups of 16, 6.3 / 7.3 / 9.8; 8191 x 8191, B = 16, 130 / 104 / 112)
   const long long groups16 = ((p.K + OUTER_TK - 1LL) / OUTER_TK) * ((p.M + 15LL) / 16) * p.groups;
