@@ -168,23 +168,6 @@ __device__ __forceinline__ void load_mn(const Mat<ST>& m, int ld, int e0, int k,
   }
 }
 
-template <int N>
-__device__ __forceinline__ void activate(int act, float (&v)[N]) {
-  switch (act) {
-    case ACT_IDENTITY: break;
-#define IPC_ACT_LOOP(A)                                  \
-  case A:                                                \
-    _Pragma("unroll") for (int i = 0; i < N; ++i) v[i] = act_t<A>(v[i]); \
-    break;
-    IPC_ACT_LOOP(ACT_RELU)
-    IPC_ACT_LOOP(ACT_TANH)
-    IPC_ACT_LOOP(ACT_SIGMOID)
-    IPC_ACT_LOOP(ACT_SILU)
-    IPC_ACT_LOOP(ACT_GELU)
-#undef IPC_ACT_LOOP
-  }
-}
-
 // The operand registers of a lane's KL values (and their lo terms: v - hi,
 // rounded), rounded like cvt: the values are pinned first, so that no product
 // behind them is folded into the conversion.

@@ -199,4 +199,22 @@ template <> struct Mfma32<bf16> {
   }
 };
 
+// N values through one branch on the activation.
+template <int N>
+__device__ __forceinline__ void activate(int act, float (&v)[N]) {
+  switch (act) {
+    case ACT_IDENTITY: break;
+#define IPC_ACT_LOOP(A)                                  \
+  case A:                                                \
+    _Pragma("unroll") for (int i = 0; i < N; ++i) v[i] = act_t<A>(v[i]); \
+    break;
+    IPC_ACT_LOOP(ACT_RELU)
+    IPC_ACT_LOOP(ACT_TANH)
+    IPC_ACT_LOOP(ACT_SIGMOID)
+    IPC_ACT_LOOP(ACT_SILU)
+    IPC_ACT_LOOP(ACT_GELU)
+#undef IPC_ACT_LOOP
+  }
+}
+
 }  // namespace ipc

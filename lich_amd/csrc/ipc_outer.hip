@@ -15,6 +15,8 @@
 // into LDS as [B][OUTER_TK].  MI355X, fp32 2048 x 2048, B = 8: 8.4 us (4.0 TB/s
 // of W), against 15.8 with W loaded after the sums, 4 bytes a lane; bf16 8192 x
 // 8192, B = 16: 79 us against 246.
+#include <type_traits>
+
 #include "ipc_device.h"
 #include "ipc_launch.h"
 
@@ -55,28 +57,44 @@ __global__ void __launch_bounds__(OUTER_TK) outer_kernel(const OuterProblem p) {
     }
   }
 
-  if (k0 + tid < K) {
-    const ST* xrow = X + (long long)(k0 + tid) * B;
-    if (B % 4 == 0 && reinterpret_cast<uintptr_t>(X) % (4 * sizeof(ST)) == 0) {
-#pragma unroll 1
-      for (int b0 = 0; b0 < B; b0 += 8) {  // two loads of 4 in flight (past B: the last 4 again)
-        float v[2][4];
+  // f(X): items of up to 8 batch values of a column, in flight together and
+  // through one branch on the activation (2, 4, 6 or 8 values, past B the last one
+  // again); a thread a column, where the block has at most 64 or 128 columns 4 or
+  // 2.  MI355X, us, 8 branches a thread and one thread a column / this: fp32 65 x
+  // 65, B = 32, tanh, 6.9 / 4.8; bf16 16 x 64, B = 18, silu, 5.7 / 4.0; fp32 512 x
+  // 4096, B = 32, gelu, 10.8 / 9.3.
+  const int kn = min(OUTER_TK, K - k0), lg = kn > 128 ? 8 : kn > 64 ? 7 : 6;
+  const int col = tid & ((1 << lg) - 1);
+  const ST* xrow = X + (long long)(k0 + col) * B;
+  const bool xvec = B % 4 == 0 && reinterpret_cast<uintptr_t>(X) % (4 * sizeof(ST)) == 0;
+  auto item = [&](auto nv, int b0) {
+    constexpr int NV = decltype(nv)::value;
+    float v[NV];
+    if (xvec && NV % 4 == 0) {
 #pragma unroll
-        for (int h = 0; h < 2; ++h) load4(xrow + min(b0 + h * 4, B - 4), v[h]);
+      for (int q = 0; q < NV / 4; ++q) {
+        float h[4];
+        load4(xrow + b0 + q * 4, h);
 #pragma unroll
-        for (int j = 0; j < 8; ++j)
-          if (b0 + j < B) xs[(b0 + j) * OUTER_LDX + tid] = act_f(p.act, v[j / 4][j % 4]);
+        for (int j = 0; j < 4; ++j) v[q * 4 + j] = h[j];
       }
     } else {
+#pragma unroll
+      for (int j = 0; j < NV; ++j) v[j] = to_f32(xrow[min(b0 + j, B - 1)]);
+    }
+    activate<NV>(p.act, v);
+#pragma unroll
+    for (int j = 0; j < NV; ++j)
+      if (b0 + j < B) xs[(b0 + j) * OUTER_LDX + col] = v[j];
+  };
+  if (col < kn) {
 #pragma unroll 1
-      for (int b0 = 0; b0 < B; b0 += 8) {  // 8 loads in flight (past B: the last value again)
-        float v[8];
-#pragma unroll
-        for (int j = 0; j < 8; ++j) v[j] = to_f32(xrow[min(b0 + j, B - 1)]);
-#pragma unroll
-        for (int j = 0; j < 8; ++j)
-          if (b0 + j < B) xs[(b0 + j) * OUTER_LDX + tid] = act_f(p.act, v[j]);
-      }
+    for (int b0 = (tid >> lg) * 8; b0 < B; b0 += (OUTER_TK >> lg) * 8) {
+      const int left = B - b0;
+      if (left > 6) item(std::integral_constant<int, 8>{}, b0);
+      else if (left > 4) item(std::integral_constant<int, 6>{}, b0);
+      else if (left > 2) item(std::integral_constant<int, 4>{}, b0);
+      else item(std::integral_constant<int, 2>{}, b0);
     }
   }
   const int mn = min(4 * RW, M - m0);
@@ -150,7 +168,7 @@ hipError_t launch_act(const void* src, void* dst, long long n, int act, int stor
 template <typename ST, int RW, bool VEC>
 static hipError_t run_outer(const OuterProblem& p, hipStream_t s) {
   const dim3 grid((p.K + OUTER_TK - 1) / OUTER_TK, (p.M + 4 * RW - 1) / (4 * RW), p.groups);
-  const size_t lds = (size_t)p.B * (OUTER_LDX + 4 * RW) * sizeof(float);  // B <= 32: at most 37,376 bytes
+  const size_t lds = (size_t)p.B * (OUTER_LDX + 4 * RW) * sizeof(float);  // B <= 32: at most 35,328 bytes
   hipLaunchKernelGGL((outer_kernel<ST, RW, VEC>), grid, dim3(OUTER_TK), lds, s, p);
   return hipGetLastError();
 }
@@ -159,7 +177,7 @@ template <typename ST>
 static hipError_t run_outer_as(const OuterProblem& p, hipStream_t s) {
   const bool vec = p.K % 4 == 0 && reinterpret_cast<uintptr_t>(p.w) % (4 * sizeof(ST)) == 0;
   // 16 rows a workgroup once that gives every CU two of them, else 8 (MI355X,
-  // us, 8 / 16 / 32 rows: fp32 2048 x 2048, B = 8, 8.3 / 7.7 / 7.7 back to back; bf16 8192 x
+  // us, 8 / 16 rows and 32, which is not instantiated: fp32 2048 x 2048, B = 8, 8.3 / 7.7 / 7.7 back to back; bf16 8192 x
   // 8192, B = 16, 116 / 79 / 68; fp16, B = 1, 47 / 41 / 44; bf16 1000 x 1531, B =
   // 5, 378 workgroups of 16, 6.3 / 7.3 / 9.8; 8191 x 8191, B = 16, 130 / 104 / 112)
   const long long groups16 = ((p.K + OUTER_TK - 1LL) / OUTER_TK) * ((p.M + 15LL) / 16) * p.groups;

@@ -36,3 +36,11 @@ def test_outer_at_tile_edges(M, K, B, groups, dt, shift):
     unit = {torch.float32: 0.0, torch.float16: 2.0 ** -11, torch.bfloat16: 2.0 ** -8}[dt]
     bound = (B + 3) * 2.0 ** -24 * mag * (1 + unit) + unit * ref.abs() + 2.0 ** -25
     assert ((w.double().cpu() - ref).abs() <= bound).all()
+
+
+@pytest.mark.parametrize("K", [1, 63, 64, 65, 128, 129, 192, 257, 320])
+@pytest.mark.parametrize("B,dt,shift", [(7, torch.float32, 0), (9, torch.float16, 0), (24, torch.bfloat16, 0),
+                                        (32, torch.float32, 0), (31, torch.float32, 1), (12, torch.float16, 1)])
+def test_outer_where_threads_share_a_column(K, B, dt, shift):
+    """Blocks of at most 64, 128 and 256 columns, whole and partial groups of 8 batch values."""
+    test_outer_at_tile_edges(21, K, B, 1, dt, shift)
