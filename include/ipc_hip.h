@@ -77,9 +77,13 @@ extern "C" {
  * tensors and, for operands read transposed, a contiguous extent that is a
  * multiple of 8; IPC_TILE_AUTO picks the 256 x 256 one whenever those hold
  * and its tiles fill every CU at least once (256 tiles or more over the
- * groups), the 256 x 128 one when they hold otherwise, and the k-chunk kernel
- * for calls of up to 256 tiles of 64 x 64 (inference update: 512), which use
- * no workspace; asking for a DMA tile
+ * groups), 512 x 64 tiles (IPC_ROUTE_DMA_512x64) for predictions whose loader
+ * evaluates tanh, sigmoid, silu or gelu (tanh: not where the 256 x 256 tiles
+ * fill the CUs) and whose rows they pad no further, the 256 x 128 one
+ * otherwise.  Calls of up to 256 tiles of 64 x 64 (inference update: 512) whose
+ * operands are below 2^31 bytes each go to the generic kernels instead: the
+ * k-chunk kernel, or the tile kernel for inference updates of more than 256
+ * such tiles and a contraction of at most 128.  Asking for a DMA tile
  * where they do not hold is IPC_ERR_CONFIG.  The autotuner
  * searches all of them per shape. */
 #define IPC_TILE_AUTO (-1)
@@ -469,6 +473,17 @@ int ipc_infer_update_ws(void* x, const void* e, const void* w_lower, const void*
                         int M, int K, int B, int groups, float gamma,
                         int storage, int operand, int act, int tile,
                         void* workspace, long long workspace_bytes, void* stream);
+/* No counterpart in the reference; a query for tests and tools.  The kernel that
+ * a standalone call of `kind` (IPC_PHASE_PRED: prediction or forward, INFER,
+ * WEIGHT with recompute) runs with these sizes, `storage` as operand type and
+ * 16-byte aligned tensors: a generic tile of the tile kernel (0-2), an LDS-DMA
+ * tile (3-6 or IPC_ROUTE_DMA_512x64), a tile of the k-chunk kernel
+ * (IPC_ROUTE_CHUNK_*), or a negative error code. */
+#define IPC_ROUTE_DMA_512x64 7
+#define IPC_ROUTE_CHUNK_16x16 16
+#define IPC_ROUTE_CHUNK_32x32 17
+#define IPC_ROUTE_CHUNK_64x64 18
+int ipc_kernel_route(int kind, int M, int K, int B, int groups, int storage, int act, int tile);
 long long ipc_s16_workspace_bytes(int kind, int act, int M, int K, int B, int groups);
 int ipc_set_s16_preactivate(int mode);
 int ipc_s16_preactivates(int kind, int act, int M, int K, int B);

@@ -260,37 +260,45 @@ int s16_auto_config(long long M, long long N, long long groups) {
   return t256 >= 256 ? IPC_TILE_DMA_256x256 - IPC_TILE_DMA_256x128 : 0;
 }
 
+// Whether an automatic call that the LDS-DMA kernel could run goes to the
+// generic kernels instead.  Few output tiles leave most CUs idle on 256 x 128
+// tiles; the k-chunk kernel then runs more and smaller ones and splits each
+// one's contraction.  It wins up to 256 tiles of 64 x 64 (prediction and weight
+// update), 512 for the inference update, whose operands both take the slower
+// transposing reads here.  MI355X, bf16, us, LDS-DMA / k-chunk: at 256 tiles
+// prediction 1024 x 4096 x 1024 relu 88 / 42, 1024^3 tanh 35 / 18, weight update
+// 1024 x 1024, B = 512, relu 17.3 / 11.7; at 512 prediction 4096 x 1024 x 512
+// relu 24 / 28, inference 2048 x 4096 x 1024 tanh 89 / 65; at 1024 inference 4096
+// x 1024 x 1024 39 / 44.  Inference updates of 257-512 tiles and a contraction of
+// 64 or 128, which use_chunk leaves to the tile kernel, are faster there than
+// here too (2048 x 128 x 1024 tanh, A_out kept, 21.1 / 18.1, K = 64 19.6 / 14.7;
+// without A_out 19.5 / 15.0, 18.7 / 11.5).  Operands past the k-chunk kernel's
+// 2^31 bytes stay (weight update 1024 x 1024, B = 2^20, 39.8 ms against 71.6 on
+// the tile kernel).
+bool generic_before_dma(const GemmProblem& q) {
+  return count_tiles(&q, 1, 64) <= (q.kind == KIND_INFER ? 512 : 256) && chunk_fits(q, 2);
+}
+
 // Kernel selection of a standalone call: returns 1 + the LDS-DMA configuration
 // (0: 256 x 128, 1: 128 x 256, 2: 128 x 128, 3: 256 x 256, S16_CFG_TALL: 512 x 64) if
 // that kernel runs it, 0 for the generic kernels, or an error.
-// `loader_act`: the activation the kernel's loader evaluates (identity: none).
-int select_tile(int tile, bool eligible, long long M, long long N, long long groups, bool infer = false,
-                int loader_act = IPC_ACT_IDENTITY) {
+int select_tile(int tile, bool eligible, const GemmProblem& q) {
   const bool dma_tile = tile >= IPC_TILE_DMA_256x128;
   if (dma_tile && !eligible)
     return fail(IPC_ERR_CONFIG,
                 "tile %d (LDS-DMA) needs 16-bit storage, a contraction that is a multiple of %d, 16-byte "
                 "aligned tensors and row lengths that are multiples of 8", tile, WIDE_BK);
   if (eligible && tile == IPC_TILE_AUTO) {
-    // Few output tiles leave most CUs idle on 256 x 128 tiles; the k-chunk
-    // kernel then runs more and smaller ones and splits each one's
-    // contraction.  It wins up to 256 tiles of 64 x 64 (prediction and weight
-    // update), 512 for the inference update, whose operands both take the
-    // slower transposing reads here.  MI355X, bf16, us, LDS-DMA / k-chunk: at
-    // 256 tiles prediction 1024 x 4096 x 1024 relu 88 / 42, 1024^3 tanh 35 /
-    // 18, weight update 1024 x 1024, B = 512, relu 17.3 / 11.7; at 512
-    // prediction 4096 x 1024 x 512 relu 24 / 28, inference 2048 x 4096 x 1024
-    // tanh 89 / 65; at 1024 inference 4096 x 1024 x 1024 39 / 44.
-    const long long t64 = ((M + 63) / 64) * ((N + 63) / 64) * groups;
-    if (t64 <= (infer ? 512 : 256)) return 0;
-    // The tall tiles where they pad no more rows than 256 x 128 ones
-    // (S16_CFG_TALL has the measurements); not for tanh, the cheapest of its
-    // activations, where the 256 x 256 tiles fill the CUs (us, 256 x 256 / tall:
-    // 8192^3 tanh 1993 / 2036, sigmoid 2454 / 2266; 4096 x 2048 x 4096 tanh 132 /
-    // 138, sigmoid 162 / 152).
-    const int cfg = s16_auto_config(M, N, groups);
-    const long long t128 = ((M + 255) / 256) * ((N + 127) / 128), tall = ((M + 511) / 512) * ((N + 63) / 64);
-    if (s16_costly(loader_act) && tall <= t128 && (cfg == 0 || loader_act != IPC_ACT_TANH)) return 1 + S16_CFG_TALL;
+    if (generic_before_dma(q)) return 0;
+    // The tall tiles, for the activations they pay for, where they pad no more
+    // rows than 256 x 128 ones (S16_CFG_TALL has the measurements); not for
+    // tanh, the cheapest of them, where the 256 x 256 tiles fill the CUs (us,
+    // 256 x 256 / tall: 8192^3 tanh 1993 / 2036, sigmoid 2454 / 2266; 4096 x 2048 x
+    // 4096 tanh 132 / 138, sigmoid 162 / 152).
+    const int cfg = s16_auto_config(q.M, q.N, q.groups);
+    const int act = q.kind == KIND_PRED || q.kind == KIND_FWD ? q.act_b : IPC_ACT_IDENTITY;
+    const long long t128 = ((q.M + 255LL) / 256) * ((q.N + 127LL) / 128), tall = ((q.M + 511LL) / 512) * ((q.N + 63LL) / 64);
+    if (s16_costly(act) && tall <= t128 && (cfg == 0 || act != IPC_ACT_TANH)) return 1 + S16_CFG_TALL;
     return 1 + cfg;
   }
   if (dma_tile) return 1 + tile - IPC_TILE_DMA_256x128;
@@ -453,7 +461,8 @@ int ipc_pred_err_ws(const void* x_upper, const void* w, const void* x_lower, voi
   TRY(check_ptr(w, "w", es));
   TRY(check_ptr(x_lower, "x_lower", es));
   TRY(check_ptr(e, "e", es));
-  const int use_dma = select_tile(tile, dma_eligible(storage, K, {x_upper, w}, {K, B}), M, B, groups, false, act);
+  const GemmProblem p = make_pf(KIND_PRED, x_upper, w, x_lower, e, M, K, B, groups, act, es);
+  const int use_dma = select_tile(tile, dma_eligible(storage, K, {x_upper, w}, {K, B}), p);
   if (use_dma < 0) return use_dma;
   if (use_dma) {
     WideProblem q{};
@@ -465,7 +474,6 @@ int ipc_pred_err_ws(const void* x_upper, const void* w, const void* x_lower, voi
     return run_s16(S16_PRED, q, groups, (long long)M * K, (long long)K * B, (long long)M * B, (long long)M * B, 0,
                    operand, act, use_dma - 1, workspace, workspace_bytes, stream, "ipc_pred_err");
   }
-  GemmProblem p = make_pf(KIND_PRED, x_upper, w, x_lower, e, M, K, B, groups, act, es);
   return launch_rc(launch_gemm(&p, 1, storage, operand, effective_split(storage, operand, split),
                                generic_tile(tile, p, storage), (hipStream_t)stream), "ipc_pred_err");
 }
@@ -488,7 +496,8 @@ int ipc_forward_ws(const void* x_upper, const void* w, void* out, int M, int K, 
   TRY(check_ptr(x_upper, "x_upper", es));
   TRY(check_ptr(w, "w", es));
   TRY(check_ptr(out, "out", es));
-  const int use_dma = select_tile(tile, dma_eligible(storage, K, {x_upper, w}, {K, B}), M, B, groups, false, act);
+  const GemmProblem p = make_pf(KIND_FWD, x_upper, w, nullptr, out, M, K, B, groups, act, es);
+  const int use_dma = select_tile(tile, dma_eligible(storage, K, {x_upper, w}, {K, B}), p);
   if (use_dma < 0) return use_dma;
   if (use_dma) {
     WideProblem q{};
@@ -500,7 +509,6 @@ int ipc_forward_ws(const void* x_upper, const void* w, void* out, int M, int K, 
     return run_s16(S16_FWD, q, groups, (long long)M * K, (long long)K * B, (long long)M * B, 0, 0, operand, act,
                    use_dma - 1, workspace, workspace_bytes, stream, "ipc_forward");
   }
-  GemmProblem p = make_pf(KIND_FWD, x_upper, w, nullptr, out, M, K, B, groups, act, es);
   return launch_rc(launch_gemm(&p, 1, storage, operand, effective_split(storage, operand, split),
                                generic_tile(tile, p, storage), (hipStream_t)stream), "ipc_forward");
 }
@@ -526,8 +534,8 @@ int ipc_infer_update_ws(void* x, const void* e, const void* w_lower, const void*
   TRY(check_ptr(w_lower, "w_lower", es));
   TRY(check_ptr(e_lower, "e_lower", es));
   if (a_out) TRY(check_ptr(a_out, "a_out", es));
-  const int use_dma = select_tile(tile, dma_eligible(storage, K, {w_lower, e_lower}, {M, B}), M, B, groups,
-                                  true);
+  const GemmProblem p = make_inf(x, e, w_lower, e_lower, a_out, M, K, B, groups, gamma, act, es);
+  const int use_dma = select_tile(tile, dma_eligible(storage, K, {w_lower, e_lower}, {M, B}), p);
   if (use_dma < 0) return use_dma;
   if (use_dma) {
     WideProblem q{};
@@ -542,7 +550,6 @@ int ipc_infer_update_ws(void* x, const void* e, const void* w_lower, const void*
                    (long long)M * B, operand, act, use_dma - 1, workspace, workspace_bytes, stream,
                    "ipc_infer_update");
   }
-  GemmProblem p = make_inf(x, e, w_lower, e_lower, a_out, M, K, B, groups, gamma, act, es);
   return launch_rc(launch_gemm(&p, 1, storage, operand, IPC_SPLIT_NONE, generic_tile(tile, p, storage),
                                (hipStream_t)stream),
                    "ipc_infer_update");
@@ -566,7 +573,8 @@ int ipc_weight_update_ws(void* w, const void* e, const void* x_upper, int M, int
   TRY(check_ptr(w, "w", es));
   TRY(check_ptr(e, "e", es));
   TRY(check_ptr(x_upper, "x_upper", es));
-  const int use_dma = select_tile(tile, dma_eligible(storage, B, {e, x_upper}, {B}), M, K, groups);
+  const GemmProblem p = make_wgt(w, e, x_upper, M, K, B, groups, alpha, recompute, act, es);
+  const int use_dma = select_tile(tile, dma_eligible(storage, B, {e, x_upper}, {B}), p);
   if (use_dma < 0) return use_dma;
   if (use_dma) {
     WideProblem q{};
@@ -580,7 +588,6 @@ int ipc_weight_update_ws(void* w, const void* e, const void* x_upper, int M, int
                    recompute ? act : IPC_ACT_IDENTITY, use_dma - 1, workspace, workspace_bytes, stream,
                    "ipc_weight_update");
   }
-  GemmProblem p = make_wgt(w, e, x_upper, M, K, B, groups, alpha, recompute, act, es);
   return launch_rc(launch_gemm(&p, 1, storage, operand, IPC_SPLIT_NONE, generic_tile(tile, p, storage),
                                (hipStream_t)stream),
                    "ipc_weight_update");
@@ -1676,6 +1683,24 @@ int ipc_wide_problem_check(int phase, int split, int fp32_w, int has_lo, int K, 
     return fail(IPC_ERR_CONFIG, "LDS-DMA GEMM problem refused on the host (phase %d, split %d, fp32 W %d, lo %d, "
                 "K %d, k-split %d)", phase, split, fp32_w, has_lo, K, ksplit);
   return ok();
+}
+
+int ipc_kernel_route(int kind, int M, int K, int B, int groups, int storage, int act, int tile) {
+  TRY(check_dtypes(storage, storage));
+  TRY(check_act(act));
+  TRY(check_dims(M, K, B, groups));
+  TRY(check_tile(tile));
+  const int es = elem_size(storage);
+  const GemmProblem p = kind == IPC_PHASE_INFER ? make_inf(nullptr, nullptr, nullptr, nullptr, nullptr, M, K, B, groups, 0.0f, act, es)
+                        : kind == IPC_PHASE_WEIGHT ? make_wgt(nullptr, nullptr, nullptr, M, K, B, groups, 0.0f, 1, act, es)
+                                                   : make_pf(KIND_PRED, nullptr, nullptr, nullptr, nullptr, M, K, B, groups, act, es);
+  // the row lengths of the operands, as the calls check them
+  const bool eligible = kind == IPC_PHASE_WEIGHT ? dma_eligible(storage, B, {}, {B})
+                        : kind == IPC_PHASE_INFER ? dma_eligible(storage, K, {}, {M, B})
+                                                  : dma_eligible(storage, K, {}, {K, B});
+  const int dma = select_tile(tile, eligible, p);
+  if (dma < 0) return dma;
+  return dma ? IPC_TILE_DMA_256x128 + dma - 1 : generic_tile(tile, p, storage);
 }
 
 int ipc_s16_preactivates(int kind, int act, int M, int K, int B) {
