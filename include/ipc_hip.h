@@ -428,35 +428,36 @@ int ipc_noalloc_set_spin_limit(int limit);
 int ipc_set_coresident_limit(int blocks);
 
 /*
- * Caller workspace of the standalone 16-bit-storage calls on the LDS-DMA
- * kernel (ipc_pred_err, ipc_forward, ipc_weight_update with recompute,
- * ipc_infer_update).
+ * Caller workspace of the standalone 16-bit-storage calls (ipc_pred_err,
+ * ipc_forward, ipc_weight_update with recompute, ipc_infer_update).
  * Their B operand f(X_upper) is activated in the loader of every row tile,
  * which for the exponential activations costs more VALU work than the tile's
  * MFMAs once there are many row tiles.  The _ws variants take a device
  * workspace (16-byte aligned, owned by the caller, `workspace_bytes` long):
  * when it holds ipc_s16_workspace_bytes(...) bytes (> 0) the call activates
- * f(X_upper) once into it, in its own launch on `stream`, and the GEMM then
- * reads it like its other operands; otherwise (NULL or too small) the
- * loader path runs.  Same bits either way.  Calls that share a workspace must
- * be ordered on one stream.  The variants without _ws are the _ws calls with
- * no workspace.  No counterpart in the reference (TileLang fuses the
- * activation into its loader and has no workspace); the library allocates
- * nothing on either path.
+ * f(X_upper) once into it, in its own launch on `stream`, and the GEMM (the
+ * LDS-DMA kernel, or for an automatic tile whichever kernel runs) then reads it
+ * like its other operands; otherwise (NULL or too small) the loader path runs.
+ * Same bits either way.  Calls that share a workspace must be ordered on one
+ * stream.  The variants without _ws are the _ws calls with no workspace.  No
+ * counterpart in the reference (TileLang fuses the activation into its loader
+ * and has no workspace); the library allocates nothing on either path.
  *
- * ipc_s16_workspace_bytes gives the bytes a call of `kind` (IPC_PHASE_PRED
+ * ipc_s16_workspace_bytes_tile gives the bytes a call of `kind` (IPC_PHASE_PRED
  * for ipc_pred_err_ws / ipc_forward_ws, IPC_PHASE_WEIGHT for a recomputing
- * ipc_weight_update_ws, IPC_PHASE_INFER for ipc_infer_update_ws) with M rows,
- * contraction K, batch B and `groups` groups uses: groups * K * B * 2 when it
- * pre-activates under the current mode (groups * (M * K + K * B) * 2 for the
- * inference update, which copies W_lower and E_lower transposed into the
- * workspace so that its GEMM reads both operands k-contiguous), else 0.  The
- * automatic rule: exp-based activations from M >= 1024 and K * B >= 2^20,
- * relu from M >= 4096 and K * B >= 2^22, never identity; the inference
- * update from M * K >= 2^26 and K * B >= 2^26.  ipc_s16_preactivates(kind,
- * act, M, K, B) reports the same decision (1 / 0).  ipc_set_s16_preactivate,
- * a tuning hook, sets the mode: -1 (default) the rule, 0 never, 1 whenever a
- * workspace is given.  Not thread-safe.
+ * ipc_weight_update_ws, IPC_PHASE_INFER for ipc_infer_update_ws) with its M, K,
+ * B, `groups`, tile id and 16-byte aligned tensors uses, 0 if it uses none:
+ * groups * K * B * 2 when it pre-activates under the current mode;
+ * groups * (M * K + K * B) * 2 for the inference update on the LDS-DMA kernel,
+ * which copies W_lower and E_lower transposed into the workspace so that its
+ * GEMM reads both operands k-contiguous.  ipc_s16_workspace_bytes is that for
+ * IPC_TILE_AUTO, and ipc_s16_preactivates whether it is more than 0 for one
+ * group.  The automatic rule: exp-based activations from M >= 1024 and K * B >=
+ * 2^20, relu from M >= 4096 and K * B >= 2^22, never identity; the inference
+ * update from M * K >= 2^26 and K * B >= 2^26, where it runs on the LDS-DMA
+ * kernel.  Generic tiles asked for by id use none.  ipc_set_s16_preactivate, a
+ * tuning hook, sets the mode: -1 (default) the rule, 0 never, 1 wherever the
+ * call could use a workspace, whatever its size.  Not thread-safe.
  */
 int ipc_pred_err_ws(const void* x_upper, const void* w, const void* x_lower, void* e,
                     int M, int K, int B, int groups,
@@ -485,6 +486,7 @@ int ipc_infer_update_ws(void* x, const void* e, const void* w_lower, const void*
 #define IPC_ROUTE_CHUNK_64x64 18
 int ipc_kernel_route(int kind, int M, int K, int B, int groups, int storage, int act, int tile);
 long long ipc_s16_workspace_bytes(int kind, int act, int M, int K, int B, int groups);
+long long ipc_s16_workspace_bytes_tile(int kind, int act, int M, int K, int B, int groups, int tile);
 int ipc_set_s16_preactivate(int mode);
 int ipc_s16_preactivates(int kind, int act, int M, int K, int B);
 

@@ -279,6 +279,49 @@ bool generic_before_dma(const GemmProblem& q) {
   return count_tiles(&q, 1, 64) <= (q.kind == KIND_INFER ? 512 : 256) && chunk_fits(q, 2);
 }
 
+// Pre-activation of a standalone call's B operand (ipc_set_s16_preactivate):
+// -1 automatic, 0 never, 1 always.
+int g_s16_preact = -1;
+
+// Whether a call evaluates its B operand f(X_upper) once instead of in the
+// loader of every row tile (the same bits: f of the stored value, one
+// rounding; then the GEMM reads the result through LDS DMA like every other
+// operand).  The automatic rule, from the per-kernel sweep on MI355X: the
+// exponential activations pay for the extra pass from 4 row tiles of 256
+// (M >= 1024) and a 2^20-element operand; relu, cheap in the loader, from 16
+// row tiles and 2^22 elements.  The inference update has no activated
+// operand; given a workspace it stores W_lower and E_lower transposed
+// instead, which pays only for the largest calls (W and E_lower of at least
+// 2^26 elements each): at 8192^3 3-8 % faster, at 8192 x 8192 x 2048 and
+// 4096^2 x 8192 3-9 % slower, the two copying passes outweighing the GEMM's
+// gain.
+bool s16_preact_rule(int mode, int act, int M, int K, long long kb) {
+  if (g_s16_preact == 0) return false;
+  if (mode == S16_INFER) return g_s16_preact > 0 || ((long long)M * K >= (1LL << 26) && kb >= (1LL << 26));
+  if (act == IPC_ACT_IDENTITY) return false;
+  if (g_s16_preact > 0) return true;
+  if (act == IPC_ACT_RELU) return M >= 4096 && kb >= (1LL << 22);
+  return M >= 1024 && kb >= (1LL << 20);
+}
+
+// Bytes of caller workspace a call uses (0 when it uses none): the groups'
+// activated B operands, 16-bit, contiguous; for the inference update on the
+// LDS-DMA kernel (`dma`) the groups' W_lower^T blocks [M][K], then their
+// E_lower^T blocks [B][K].  The generic kernels read an activated operand like
+// any other (the same bits as activating it in their loaders), gain nothing from
+// transposed ones (inference 1024 x 65536 x 1024, MI355X: 465 us as it is, 1067
+// on the LDS-DMA kernel with both copied), and as explicit tiles take none.
+// MI355X, bf16, us, k-chunk kernel alone / lent a workspace, LDS-DMA kernel lent
+// one: 1024^3 tanh 19.4 / 14.3, 25.4; 4096 x 4096 x 256 silu 87.7 / 44.1, 65.2; 4096
+// x 8192 x 256 silu 172 / 111, 117; 1024 x 8192 x 256 gelu 73 / 44, 117; weight
+// update 1024 x 1024, B = 8192, sigmoid 163 / 90, 129; only 8192 x 8192 x 128 (silu
+// 177 / 126, 116) would gain on the LDS-DMA kernel.
+long long s16_workspace_need(int mode, int act, const GemmProblem& q, int tile, bool dma) {
+  if (!s16_preact_rule(mode, act, q.M, q.K, q.b_gs)) return 0;
+  if (!dma && (mode == S16_INFER || tile != IPC_TILE_AUTO)) return 0;
+  return mode == S16_INFER ? (long long)q.groups * (q.a_gs + q.b_gs) * 2 : (long long)q.groups * q.b_gs * 2;
+}
+
 // Kernel selection of a standalone call: returns 1 + the LDS-DMA configuration
 // (0: 256 x 128, 1: 128 x 256, 2: 128 x 128, 3: 256 x 256, S16_CFG_TALL: 512 x 64) if
 // that kernel runs it, 0 for the generic kernels, or an error.
@@ -328,53 +371,18 @@ std::vector<WideProblem> s16_groups(const WideProblem& q, int groups, long long 
   return v;
 }
 
-// Pre-activation of a standalone call's B operand (ipc_set_s16_preactivate):
-// -1 automatic, 0 never, 1 always.
-int g_s16_preact = -1;
-
-// Whether a call evaluates its B operand f(X_upper) once instead of in the
-// loader of every row tile (the same bits: f of the stored value, one
-// rounding; then the GEMM reads the result through LDS DMA like every other
-// operand).  The automatic rule, from the per-kernel sweep on MI355X: the
-// exponential activations pay for the extra pass from 4 row tiles of 256
-// (M >= 1024) and a 2^20-element operand; relu, cheap in the loader, from 16
-// row tiles and 2^22 elements.  The inference update has no activated
-// operand; given a workspace it stores W_lower and E_lower transposed
-// instead, which pays only for the largest calls (W and E_lower of at least
-// 2^26 elements each): at 8192^3 3-8 % faster, at 8192 x 8192 x 2048 and
-// 4096^2 x 8192 3-9 % slower, the two copying passes outweighing the GEMM's
-// gain.
-bool s16_preact_rule(int mode, int act, int M, int K, long long kb) {
-  if (g_s16_preact == 0) return false;
-  if (mode == S16_INFER) return g_s16_preact > 0 || ((long long)M * K >= (1LL << 26) && kb >= (1LL << 26));
-  if (act == IPC_ACT_IDENTITY) return false;
-  if (g_s16_preact > 0) return true;
-  if (act == IPC_ACT_RELU) return M >= 4096 && kb >= (1LL << 22);
-  return M >= 1024 && kb >= (1LL << 20);
-}
-
-// Bytes of caller workspace a call uses (0 when the rule says it does not
-// use one): the groups' activated B operands, 16-bit, contiguous; for the
-// inference update the groups' W_lower^T blocks [M][K], then their
-// E_lower^T blocks [B][K].
-long long s16_workspace_need(int mode, int act, int M, int K, long long kb, int groups) {
-  if (!s16_preact_rule(mode, act, M, K, kb)) return 0;
-  return mode == S16_INFER ? (long long)groups * ((long long)M * K + kb) * 2 : (long long)groups * kb * 2;
-}
-
-// A standalone call on the LDS-DMA kernel.  With a caller workspace of at
-// least s16_workspace_need bytes the B operand is activated once into it
+// A standalone call on the LDS-DMA kernel.  With a workspace lent (at
+// least s16_workspace_need bytes) the B operand is activated once into it
 // (an elementwise launch) and the GEMM reads it like the other operands, or,
 // for the inference update, both operands are copied transposed into it;
 // otherwise every row tile activates its B block in its loader and the
 // inference update reads its operands transposed from LDS.  The library
 // allocates nothing either way.
 int run_s16(int mode, const WideProblem& q, int groups, long long a_gs, long long b_gs, long long o_gs,
-            long long x_gs, long long o2_gs, int operand, int act, int cfg, void* workspace, long long ws_bytes,
+            long long x_gs, long long o2_gs, int operand, int act, int cfg, void* workspace, bool lent,
             void* stream, const char* what) {
   hipStream_t s = (hipStream_t)stream;
-  const long long need = s16_workspace_need(mode, act, q.M, q.K, b_gs, groups);
-  if (need > 0 && workspace && ws_bytes >= need) {
+  if (lent) {
     if (cfg == S16_CFG_TALL) cfg = s16_auto_config(q.M, q.N, groups);  // f(X) no longer in the loader
     WideProblem qa = q;
     if (mode == S16_INFER) {
@@ -409,6 +417,26 @@ int run_s16(int mode, const WideProblem& q, int groups, long long a_gs, long lon
   }
   const std::vector<WideProblem> v = s16_groups(q, groups, a_gs, b_gs, o_gs, x_gs, o2_gs);
   return launch_rc(launch_s16(mode, v.data(), groups, operand, act, cfg, s), what);
+}
+
+// Whether the caller lends the workspace that a call uses.
+bool ws_lent(int storage, int mode, int act, const GemmProblem& q, int tile, bool dma, const void* workspace,
+             long long ws_bytes) {
+  const long long need = storage == IPC_DT_F32 ? 0 : s16_workspace_need(mode, act, q, tile, dma);
+  return need > 0 && workspace && ws_bytes >= need;
+}
+
+// A 16-bit call on the generic kernels: with a workspace lent, B activated into it first.
+int run_generic(GemmProblem q, int storage, int operand, int split, int tile, bool lent, void* workspace, void* stream,
+                const char* what) {
+  if (lent) {
+    TRY(launch_rc(launch_s16_activate(q.b, workspace, (long long)q.groups * q.b_gs, operand, q.act_b, (hipStream_t)stream),
+                  what));
+    q.b = workspace;
+    q.act_b = IPC_ACT_IDENTITY;
+    q.vec_b = vec_ok(workspace, q.ldb, 2);
+  }
+  return launch_rc(launch_gemm(&q, 1, storage, operand, split, generic_tile(tile, q, storage), (hipStream_t)stream), what);
 }
 
 int check_workspace(const void* workspace, long long ws_bytes) {
@@ -464,6 +492,8 @@ int ipc_pred_err_ws(const void* x_upper, const void* w, const void* x_lower, voi
   const GemmProblem p = make_pf(KIND_PRED, x_upper, w, x_lower, e, M, K, B, groups, act, es);
   const int use_dma = select_tile(tile, dma_eligible(storage, K, {x_upper, w}, {K, B}), p);
   if (use_dma < 0) return use_dma;
+  const bool lent =
+      ws_lent(storage, S16_PRED, act, p, tile, use_dma > 0, workspace, workspace_bytes);
   if (use_dma) {
     WideProblem q{};
     q.M = M; q.N = B; q.K = K;
@@ -472,10 +502,9 @@ int ipc_pred_err_ws(const void* x_upper, const void* w, const void* x_lower, voi
     q.out = e; q.ldo = B; q.aux = x_lower; q.ldx = B;
     q.vec = B % 4 == 0 && al8(e) && al8(x_lower);
     return run_s16(S16_PRED, q, groups, (long long)M * K, (long long)K * B, (long long)M * B, (long long)M * B, 0,
-                   operand, act, use_dma - 1, workspace, workspace_bytes, stream, "ipc_pred_err");
+                   operand, act, use_dma - 1, workspace, lent, stream, "ipc_pred_err");
   }
-  return launch_rc(launch_gemm(&p, 1, storage, operand, effective_split(storage, operand, split),
-                               generic_tile(tile, p, storage), (hipStream_t)stream), "ipc_pred_err");
+  return run_generic(p, storage, operand, effective_split(storage, operand, split), tile, lent, workspace, stream, "ipc_pred_err");
 }
 
 int ipc_forward(const void* x_upper, const void* w, void* out, int M, int K, int B, int groups, int storage,
@@ -499,6 +528,8 @@ int ipc_forward_ws(const void* x_upper, const void* w, void* out, int M, int K, 
   const GemmProblem p = make_pf(KIND_FWD, x_upper, w, nullptr, out, M, K, B, groups, act, es);
   const int use_dma = select_tile(tile, dma_eligible(storage, K, {x_upper, w}, {K, B}), p);
   if (use_dma < 0) return use_dma;
+  const bool lent =
+      ws_lent(storage, S16_FWD, act, p, tile, use_dma > 0, workspace, workspace_bytes);
   if (use_dma) {
     WideProblem q{};
     q.M = M; q.N = B; q.K = K;
@@ -507,10 +538,9 @@ int ipc_forward_ws(const void* x_upper, const void* w, void* out, int M, int K, 
     q.out = out; q.ldo = B;
     q.vec = B % 4 == 0 && al8(out);
     return run_s16(S16_FWD, q, groups, (long long)M * K, (long long)K * B, (long long)M * B, 0, 0, operand, act,
-                   use_dma - 1, workspace, workspace_bytes, stream, "ipc_forward");
+                   use_dma - 1, workspace, lent, stream, "ipc_forward");
   }
-  return launch_rc(launch_gemm(&p, 1, storage, operand, effective_split(storage, operand, split),
-                               generic_tile(tile, p, storage), (hipStream_t)stream), "ipc_forward");
+  return run_generic(p, storage, operand, effective_split(storage, operand, split), tile, lent, workspace, stream, "ipc_forward");
 }
 
 int ipc_infer_update(void* x, const void* e, const void* w_lower, const void* e_lower, void* a_out, int M,
@@ -537,6 +567,8 @@ int ipc_infer_update_ws(void* x, const void* e, const void* w_lower, const void*
   const GemmProblem p = make_inf(x, e, w_lower, e_lower, a_out, M, K, B, groups, gamma, act, es);
   const int use_dma = select_tile(tile, dma_eligible(storage, K, {w_lower, e_lower}, {M, B}), p);
   if (use_dma < 0) return use_dma;
+  const bool lent =
+      ws_lent(storage, S16_INFER, act, p, tile, use_dma > 0, workspace, workspace_bytes);
   if (use_dma) {
     WideProblem q{};
     q.M = M; q.N = B; q.K = K;
@@ -547,12 +579,10 @@ int ipc_infer_update_ws(void* x, const void* e, const void* w_lower, const void*
     q.scal = gamma;
     q.vec = B % 4 == 0 && al8(x) && al8(e) && al8(a_out);
     return run_s16(S16_INFER, q, groups, (long long)K * M, (long long)K * B, (long long)M * B, (long long)M * B,
-                   (long long)M * B, operand, act, use_dma - 1, workspace, workspace_bytes, stream,
+                   (long long)M * B, operand, act, use_dma - 1, workspace, lent, stream,
                    "ipc_infer_update");
   }
-  return launch_rc(launch_gemm(&p, 1, storage, operand, IPC_SPLIT_NONE, generic_tile(tile, p, storage),
-                               (hipStream_t)stream),
-                   "ipc_infer_update");
+  return run_generic(p, storage, operand, IPC_SPLIT_NONE, tile, lent, workspace, stream, "ipc_infer_update");
 }
 
 int ipc_weight_update(void* w, const void* e, const void* x_upper, int M, int K, int B, int groups,
@@ -576,6 +606,8 @@ int ipc_weight_update_ws(void* w, const void* e, const void* x_upper, int M, int
   const GemmProblem p = make_wgt(w, e, x_upper, M, K, B, groups, alpha, recompute, act, es);
   const int use_dma = select_tile(tile, dma_eligible(storage, B, {e, x_upper}, {B}), p);
   if (use_dma < 0) return use_dma;
+  const bool lent =
+      ws_lent(storage, S16_WEIGHT, recompute ? act : IPC_ACT_IDENTITY, p, tile, use_dma > 0, workspace, workspace_bytes);
   if (use_dma) {
     WideProblem q{};
     q.M = M; q.N = K; q.K = B;
@@ -585,12 +617,10 @@ int ipc_weight_update_ws(void* w, const void* e, const void* x_upper, int M, int
     q.scal = alpha;
     q.vec = K % 4 == 0 && al8(w);
     return run_s16(S16_WEIGHT, q, groups, (long long)M * B, (long long)K * B, (long long)M * K, 0, 0, operand,
-                   recompute ? act : IPC_ACT_IDENTITY, use_dma - 1, workspace, workspace_bytes, stream,
+                   recompute ? act : IPC_ACT_IDENTITY, use_dma - 1, workspace, lent, stream,
                    "ipc_weight_update");
   }
-  return launch_rc(launch_gemm(&p, 1, storage, operand, IPC_SPLIT_NONE, generic_tile(tile, p, storage),
-                               (hipStream_t)stream),
-                   "ipc_weight_update");
+  return run_generic(p, storage, operand, IPC_SPLIT_NONE, tile, lent, workspace, stream, "ipc_weight_update");
 }
 
 int ipc_weight_update_outer(void* w, const void* e, const void* x_upper, int M, int K, int B, int groups,
@@ -1685,33 +1715,55 @@ int ipc_wide_problem_check(int phase, int split, int fp32_w, int has_lo, int K, 
   return ok();
 }
 
+}  // extern "C"
+
+namespace {
+// A standalone call with these sizes and 16-byte aligned tensors: its problem
+// and whether its row lengths suit the LDS-DMA kernel.
+GemmProblem shape_of(int kind, int M, int K, int B, int groups, int storage, int act, bool* eligible) {
+  const int es = elem_size(storage);
+  if (kind == IPC_PHASE_INFER) {
+    *eligible = dma_eligible(storage, K, {}, {M, B});
+    return make_inf(nullptr, nullptr, nullptr, nullptr, nullptr, M, K, B, groups, 0.0f, act, es);
+  }
+  if (kind == IPC_PHASE_WEIGHT) {
+    *eligible = dma_eligible(storage, B, {}, {B});
+    return make_wgt(nullptr, nullptr, nullptr, M, K, B, groups, 0.0f, 1, act, es);
+  }
+  *eligible = dma_eligible(storage, K, {}, {K, B});
+  return make_pf(KIND_PRED, nullptr, nullptr, nullptr, nullptr, M, K, B, groups, act, es);
+}
+}  // namespace
+
+extern "C" {
+
 int ipc_kernel_route(int kind, int M, int K, int B, int groups, int storage, int act, int tile) {
   TRY(check_dtypes(storage, storage));
   TRY(check_act(act));
   TRY(check_dims(M, K, B, groups));
   TRY(check_tile(tile));
-  const int es = elem_size(storage);
-  const GemmProblem p = kind == IPC_PHASE_INFER ? make_inf(nullptr, nullptr, nullptr, nullptr, nullptr, M, K, B, groups, 0.0f, act, es)
-                        : kind == IPC_PHASE_WEIGHT ? make_wgt(nullptr, nullptr, nullptr, M, K, B, groups, 0.0f, 1, act, es)
-                                                   : make_pf(KIND_PRED, nullptr, nullptr, nullptr, nullptr, M, K, B, groups, act, es);
-  // the row lengths of the operands, as the calls check them
-  const bool eligible = kind == IPC_PHASE_WEIGHT ? dma_eligible(storage, B, {}, {B})
-                        : kind == IPC_PHASE_INFER ? dma_eligible(storage, K, {}, {M, B})
-                                                  : dma_eligible(storage, K, {}, {K, B});
+  bool eligible = false;
+  const GemmProblem p = shape_of(kind, M, K, B, groups, storage, act, &eligible);
   const int dma = select_tile(tile, eligible, p);
   if (dma < 0) return dma;
   return dma ? IPC_TILE_DMA_256x128 + dma - 1 : generic_tile(tile, p, storage);
 }
 
 int ipc_s16_preactivates(int kind, int act, int M, int K, int B) {
-  const int mode = kind == IPC_PHASE_PRED ? S16_PRED : kind == IPC_PHASE_WEIGHT ? S16_WEIGHT : S16_INFER;
-  return s16_preact_rule(mode, act, M, K, (long long)K * B) ? 1 : 0;
+  return ipc_s16_workspace_bytes(kind, act, M, K, B, 1) > 0 ? 1 : 0;
 }
 
 long long ipc_s16_workspace_bytes(int kind, int act, int M, int K, int B, int groups) {
-  if (M < 1 || K < 1 || B < 1 || groups < 1) return 0;
+  return ipc_s16_workspace_bytes_tile(kind, act, M, K, B, groups, IPC_TILE_AUTO);
+}
+
+long long ipc_s16_workspace_bytes_tile(int kind, int act, int M, int K, int B, int groups, int tile) {
+  if (M < 1 || K < 1 || B < 1 || groups < 1 || tile < IPC_TILE_AUTO || tile >= IPC_TILE_COUNT) return 0;
   const int mode = kind == IPC_PHASE_PRED ? S16_PRED : kind == IPC_PHASE_WEIGHT ? S16_WEIGHT : S16_INFER;
-  return s16_workspace_need(mode, act, M, K, (long long)K * B, groups);
+  bool eligible = false;
+  const GemmProblem p = shape_of(kind, M, K, B, groups, IPC_DT_BF16, act, &eligible);
+  const int dma = select_tile(tile, eligible, p);
+  return dma < 0 ? 0 : s16_workspace_need(mode, act, p, tile, dma > 0);
 }
 
 int ipc_set_s16_preactivate(int mode) {

@@ -118,13 +118,14 @@ class _Kernel:
     @property
     def workspace_bytes(self) -> int:
         """Bytes of caller workspace that let a call evaluate f(X_upper) once
-        instead of in every row tile's loader, or, for the inference update,
-        copy its operands transposed (0: the call never uses one).
-        Only 16-bit storage on the LDS-DMA kernel uses it; the library itself
-        allocates nothing."""
+        instead of in every row tile's loader, or, for the inference update on
+        the LDS-DMA kernel, copy its operands transposed (0: the call never
+        uses one).  Only 16-bit storage uses one; the library itself allocates
+        nothing."""
         if self._ws_kind < 0 or self.storage == nat.DT_F32:
             return 0
-        return int(nat.lib().ipc_s16_workspace_bytes(self._ws_kind, self.act, self.M, self.K, self.B, self.groups))
+        return int(nat.lib().ipc_s16_workspace_bytes_tile(self._ws_kind, self.act, self.M, self.K, self.B, self.groups,
+                                                          self.tile))
 
     def new_workspace(self, device=None) -> torch.Tensor | None:
         """A caller-owned workspace of ``workspace_bytes`` (None when the call

@@ -26,3 +26,25 @@ def route(kind, M, K, B, groups=1, st="bf16", act="relu", tile=-1):
 ])
 def test_automatic_16_bit_calls(kind, M, K, B, want):
     assert route(kind, M, K, B) in want
+
+
+def test_workspace_bytes_are_those_of_the_call():
+    """0 exactly where the call would not use a workspace (0 used to be promised
+    that, and more than 0 asked for, by calls of few tiles that ignored it)."""
+    lib, tanh = nat.lib(), nat.act_code("tanh")
+    wb, wt = lib.ipc_s16_workspace_bytes, lib.ipc_s16_workspace_bytes_tile
+    assert wb(PRED, tanh, 1024, 1024, 1024, 1) == 1024 * 1024 * 2  # the k-chunk kernel reads it
+    assert wb(PRED, tanh, 1024, 1031, 1025, 1) == 1031 * 1025 * 2
+    for tile in range(7):  # explicit tiles: the LDS-DMA kernel's only
+        assert wt(PRED, tanh, 1024, 1024, 1024, 1, tile) == (1024 * 1024 * 2 if tile >= 3 else 0)
+    assert wt(WEIGHT, tanh, 1024, 1024, 1031, 1, 3) == 0  # a tile the call would be refused for
+    # the inference update: only where it runs on the LDS-DMA kernel
+    assert wb(INFER, tanh, 1024, 65536, 1024, 1) == 0 and wt(INFER, tanh, 1024, 65536, 1024, 1, 3) == 2 * (1 << 27)
+    assert lib.ipc_s16_preactivates(INFER, tanh, 1024, 65536, 1024) == 0
+    try:
+        assert lib.ipc_set_s16_preactivate(1) == 0
+        assert wb(PRED, tanh, 64, 784, 128, 1) == 784 * 128 * 2 and wb(INFER, tanh, 64, 64, 64, 1) == 0
+        assert wb(INFER, tanh, 4096, 4096, 1024, 1) == 2 * (4096 * 4096 + 4096 * 1024)
+        assert lib.ipc_set_s16_preactivate(0) == 0 and wb(PRED, tanh, 8192, 8192, 8192, 1) == 0
+    finally:
+        lib.ipc_set_s16_preactivate(-1)
