@@ -60,12 +60,12 @@ extern "C" {
 #define IPC_ACT_GELU 5
 
 /* tile configurations of the MFMA GEMM family; IPC_TILE_AUTO picks by shape.
- * The generic ids 0-2 name a small, a middle and a large output tile.  With
- * fp32 storage they run on the k-chunk kernel (16 x 16, 32 x 32, 64 x 64
- * tiles, the contraction split over a workgroup's waves; the automatic tile
- * where that is larger) wherever that is the faster one, else on the tile kernel (32 x 32, 64 x 64, 128 x 128); the bits
- * depend on the kernel, not on the tile.  With 16-bit storage the ids name the
- * tile kernel, whose k order is the LDS-DMA kernel's.
+ * The generic ids 0-2 name 32 x 32, 64 x 64 and 128 x 128 output tiles.  With
+ * fp32 storage they run on the k-chunk kernel (the contraction split over a
+ * workgroup's waves; 128 x 128 names its largest tile, 64 x 64) wherever that is
+ * the faster one, else on the tile kernel; the bits depend on the kernel, not on
+ * the tile.  With 16-bit storage the ids name the tile kernel, whose k order is
+ * the LDS-DMA kernel's.  IPC_TILE_AUTO also picks the k-chunk kernel's 16 x 16.
  * IPC_TILE_DMA_* are the LDS-DMA kernel (operands streamed HBM -> LDS without
  * VGPR staging, transposed operands read with the LDS transpose read) in
  * four tile configurations: 256 x 128, 128 x 256,

@@ -149,17 +149,19 @@ bool use_chunk(const GemmProblem* q, int n, int esize) {
 }
 
 // Tile of such a launch.  `tile`: IPC_TILE_AUTO, or a generic tile id, which
-// names the small, middle or large tile of either kernel, in the k-chunk kernel
-// the automatic one where that is larger (neither kernel's bits depend on the
-// tile).  Automatic: the largest tile that gives the 256
-// CUs about a workgroup each; a larger tile reads its operands less often, a
-// smaller one starts more waves.  MI355X, k-chunk kernel, fp32 storage, 16-bit
-// operands, us for 16 / 32 / 64: 512 x 512 x 2000 split 2 (256 large tiles)
+// names 32 x 32, 64 x 64 or 128 x 128 tiles; the k-chunk kernel's largest is 64 x 64
+// (neither kernel's bits depend on the tile).  Automatic: the largest tile that
+// gives the 256 CUs about a workgroup each; a larger tile reads its operands less
+// often, a smaller one starts more waves.  MI355X, k-chunk kernel, fp32 storage,
+// 16-bit operands, us for 16 / 32 / 64: 512 x 512 x 2000 split 2 (256 large tiles)
 // 29.7 / 23.2 / 16.6, 512 x 784 x 256 (32 large, 128 middle tiles) 8.9 / 11.1
 // / 17.6, 1024^3 54 / 41 / 19.7.
 int pick_tile(int tile, const GemmProblem* q, int n, bool chunk) {
   const long long t64 = count_tiles(q, n, 64);
-  if (chunk) return TILE_CHUNK_16 + std::max(tile, t64 >= 192 ? 2 : count_tiles(q, n, 32) >= 256 ? 1 : 0);
+  if (chunk) {
+    if (tile != IPC_TILE_AUTO) return tile == IPC_TILE_32x32 ? TILE_CHUNK_32 : TILE_CHUNK_64;
+    return t64 >= 192 ? TILE_CHUNK_64 : count_tiles(q, n, 32) >= 256 ? TILE_CHUNK_32 : TILE_CHUNK_16;
+  }
   if (tile != IPC_TILE_AUTO) return tile;
   return count_tiles(q, n, 128) >= 512 ? IPC_TILE_128x128 : t64 >= 64 ? IPC_TILE_64x64 : IPC_TILE_32x32;
 }
@@ -906,7 +908,8 @@ long long resident_eligible(int L, const int* dims, int B, int operand, int spli
 }
 
 // Kernels and tiles of the phased launches (tiles as set by ipc_plan_set_tiles
-// or automatic).  A net that the wide path could run as well keeps the tile
+// or automatic; with 16-bit storage a tile set by id is the tile kernel's, as in
+// the standalone calls).  A net that the wide path could run as well keeps the tile
 // kernel: its k order is the wide path's, so the two paths' 16-bit operands
 // round alike and their states agree to fp32 rounding over many steps.
 void pick_phase_tiles(ipc_plan* plan) {
@@ -914,7 +917,8 @@ void pick_phase_tiles(ipc_plan* plan) {
                      !narrow_eligible(plan->L, plan->dims.data(), plan->storage, plan->operand, plan->split);
   const int es = elem_size(plan->storage), *t = plan->tile_override;
   auto pick = [&](int want, const std::vector<GemmProblem>& v) {
-    return pick_tile(want, v.data(), (int)v.size(), !chain && use_chunk(v.data(), (int)v.size(), es));
+    const bool chunk = !chain && (es == 4 || want == IPC_TILE_AUTO) && use_chunk(v.data(), (int)v.size(), es);
+    return pick_tile(want, v.data(), (int)v.size(), chunk);
   };
   plan->tile_pred = pick(t[0], plan->pred);
   plan->tile_infer = pick(t[1], plan->infer);

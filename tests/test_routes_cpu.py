@@ -48,3 +48,11 @@ def test_workspace_bytes_are_those_of_the_call():
         assert lib.ipc_set_s16_preactivate(0) == 0 and wb(PRED, tanh, 8192, 8192, 8192, 1) == 0
     finally:
         lib.ipc_set_s16_preactivate(-1)
+
+
+@pytest.mark.parametrize("kind", [PRED, INFER, WEIGHT])
+@pytest.mark.parametrize("M,K,B", [(64, 784, 128), (512, 784, 256), (512, 512, 2000), (1024, 1024, 1024)])
+def test_generic_tiles_run_as_asked_for(kind, M, K, B):
+    assert [route(kind, M, K, B, st="fp32", tile=t) for t in (0, 1, 2)] == [17, 18, 18]  # k-chunk: 64 x 64 at most
+    assert [route(kind, M, K, B, st="fp16", tile=t) for t in (0, 1, 2)] == [0, 1, 2]     # the tile kernel
+    assert route(kind, 4096, 4096, 2048, st="fp32", tile=0) == (17 if kind == INFER else 0)
