@@ -133,8 +133,17 @@ long long count_tiles(const GemmProblem* q, int n, int e) {
 //   54; inference 4096 x 64 x 2048 29.7 / 54.8, 2048 x 256 x 2048 32 / 35.6,
 //   2048 x 384 x 2048 41.6 / 37.5; at 256 tiles of 64 x 64 the k-chunk kernel is
 //   ahead even at one chunk, inference 1024 x 100 x 1024 12.0 / 8.6, at 512 from
-//   two on, 2048 x 200 x 1024 20.9 / 17.3).
-bool use_chunk(const GemmProblem* q, int n, int esize) {
+//   two on, 2048 x 200 x 1024 20.9 / 17.3;
+// * 1,024 tiles or more of 5 to 11 chunks (a round of a workgroup's 8 waves that
+//   is not full) whose loader evaluates an activation that costs as much as the
+//   products, which the k-chunk kernel's 64 x 64 tiles do up to twice as often
+//   and within the same waves: sigmoid and silu, with fp32 operands also tanh and
+//   gelu (prediction 4096 x 780 x 2048, fp32 storage, fp16 operands, sigmoid 121 /
+//   159, bf16 storage 700 x 1300 x 7000 sigmoid 150 / 170, tanh 4096 x 780 x 2048
+//   153 / 133; fp32 operands 2048 x 780 x 2048 tanh 108 / 114, weight update 700 x
+//   7000, B = 780, gelu 141 / 168; at 8 chunks bf16 storage 2048 x 900 x 2048
+//   sigmoid 93 / 84).
+bool use_chunk(const GemmProblem* q, int n, int esize, bool fp32_operands, int split) {
   int kmax = 0;
   for (int i = 0; i < n; ++i) {
     if (!chunk_fits(q[i], esize)) return false;
@@ -145,6 +154,14 @@ bool use_chunk(const GemmProblem* q, int n, int esize) {
   const long long t64 = count_tiles(q, n, 64);
   if (t64 > 256 && kmax <= 128) return false;
   if (t64 > 512 && kmax <= (infer ? 256 : 512)) return false;
+  if (n == 1 && !infer && t64 >= (split == IPC_SPLIT_WX ? 2048 : 1024) && kmax <= 1408) {
+    const bool full = kmax > 896 && kmax <= 1024;  // 8 chunks
+    // rows of odd length cost the tile kernel more than this one with 16-bit operands
+    const bool rows = fp32_operands || (esize == 4 && q[0].kind != KIND_WEIGHT) || (q[0].vec_a && q[0].vec_b);
+    const int act = q[0].act_b;
+    if (rows && (act == IPC_ACT_SIGMOID || act == IPC_ACT_SILU) && (esize == 4 || !full)) return false;
+    if (rows && (act == IPC_ACT_TANH || act == IPC_ACT_GELU) && fp32_operands && !full) return false;
+  }
   return !(esize == 4 && !infer && kmax >= 1024 && count_tiles(q, n, 128) >= 512);
 }
 
@@ -353,9 +370,9 @@ int select_tile(int tile, bool eligible, const GemmProblem& q) {
 // Tile of a standalone call that the LDS-DMA kernel does not run (`tile` as
 // asked for).  A generic tile asked for by id with 16-bit storage is the tile
 // kernel's, whose k order (and so every bit) is the LDS-DMA kernel's.
-int generic_tile(int tile, const GemmProblem& q, int storage) {
+int generic_tile(int tile, const GemmProblem& q, int storage, int operand, int split) {
   if (storage != IPC_DT_F32 && tile != IPC_TILE_AUTO) return tile;
-  return pick_tile(tile, &q, 1, use_chunk(&q, 1, elem_size(storage)));
+  return pick_tile(tile, &q, 1, use_chunk(&q, 1, elem_size(storage), operand == IPC_DT_F32, split));
 }
 
 // One WideProblem per group of a standalone 16-bit call.
@@ -428,9 +445,11 @@ bool ws_lent(int storage, int mode, int act, const GemmProblem& q, int tile, boo
   return need > 0 && workspace && ws_bytes >= need;
 }
 
-// A 16-bit call on the generic kernels: with a workspace lent, B activated into it first.
+// A call on the generic kernels: with a workspace lent, B activated into it first
+// (the kernel is the one that runs without, whose bits the result has).
 int run_generic(GemmProblem q, int storage, int operand, int split, int tile, bool lent, void* workspace, void* stream,
                 const char* what) {
+  const int run = generic_tile(tile, q, storage, operand, split);
   if (lent) {
     TRY(launch_rc(launch_s16_activate(q.b, workspace, (long long)q.groups * q.b_gs, operand, q.act_b, (hipStream_t)stream),
                   what));
@@ -438,7 +457,7 @@ int run_generic(GemmProblem q, int storage, int operand, int split, int tile, bo
     q.act_b = IPC_ACT_IDENTITY;
     q.vec_b = vec_ok(workspace, q.ldb, 2);
   }
-  return launch_rc(launch_gemm(&q, 1, storage, operand, split, generic_tile(tile, q, storage), (hipStream_t)stream), what);
+  return launch_rc(launch_gemm(&q, 1, storage, operand, split, run, (hipStream_t)stream), what);
 }
 
 int check_workspace(const void* workspace, long long ws_bytes) {
@@ -917,7 +936,9 @@ void pick_phase_tiles(ipc_plan* plan) {
                      !narrow_eligible(plan->L, plan->dims.data(), plan->storage, plan->operand, plan->split);
   const int es = elem_size(plan->storage), *t = plan->tile_override;
   auto pick = [&](int want, const std::vector<GemmProblem>& v) {
-    const bool chunk = !chain && (es == 4 || want == IPC_TILE_AUTO) && use_chunk(v.data(), (int)v.size(), es);
+    const int split = v.empty() || v[0].kind != KIND_PRED ? IPC_SPLIT_NONE : plan->split;
+    const bool chunk = !chain && (es == 4 || want == IPC_TILE_AUTO) &&
+                       use_chunk(v.data(), (int)v.size(), es, plan->operand == IPC_DT_F32, split);
     return pick_tile(want, v.data(), (int)v.size(), chunk);
   };
   plan->tile_pred = pick(t[0], plan->pred);
@@ -1750,7 +1771,7 @@ int ipc_kernel_route(int kind, int M, int K, int B, int groups, int storage, int
   const GemmProblem p = shape_of(kind, M, K, B, groups, storage, act, &eligible);
   const int dma = select_tile(tile, eligible, p);
   if (dma < 0) return dma;
-  return dma ? IPC_TILE_DMA_256x128 + dma - 1 : generic_tile(tile, p, storage);
+  return dma ? IPC_TILE_DMA_256x128 + dma - 1 : generic_tile(tile, p, storage, storage, IPC_SPLIT_NONE);
 }
 
 int ipc_s16_preactivates(int kind, int act, int M, int K, int B) {

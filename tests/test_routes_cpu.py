@@ -56,3 +56,16 @@ def test_generic_tiles_run_as_asked_for(kind, M, K, B):
     assert [route(kind, M, K, B, st="fp32", tile=t) for t in (0, 1, 2)] == [17, 18, 18]  # k-chunk: 64 x 64 at most
     assert [route(kind, M, K, B, st="fp16", tile=t) for t in (0, 1, 2)] == [0, 1, 2]     # the tile kernel
     assert route(kind, 4096, 4096, 2048, st="fp32", tile=0) == (17 if kind == INFER else 0)
+
+
+@pytest.mark.parametrize("kind,M,K,B,st,act,chunk", [
+    (PRED, 4096, 780, 2048, "fp32", "sigmoid", False), (PRED, 4096, 780, 2048, "fp32", "relu", True),
+    (PRED, 4096, 900, 2048, "fp16", "silu", True), (PRED, 4096, 780, 2048, "fp16", "silu", False),
+    (PRED, 4096, 780, 2048, "fp16", "tanh", True), (PRED, 4096, 780, 2048, "fp32", "tanh", False),
+    (PRED, 1920, 780, 2048, "fp32", "sigmoid", True), (PRED, 4096, 1412, 2048, "fp16", "sigmoid", True),
+    (INFER, 4096, 780, 2048, "fp32", "sigmoid", True),
+    (WEIGHT, 2048, 4096, 780, "fp32", "gelu", False), (WEIGHT, 2048, 4096, 780, "fp16", "gelu", True),
+])
+def test_many_tiles_of_a_partly_filled_round(kind, M, K, B, st, act, chunk):
+    """Loaders with a costly activation: the tile kernel, which the k-chunk kernel had slowed down."""
+    assert (route(kind, M, K, B, st=st, act=act) in CHUNK) == chunk
