@@ -172,7 +172,11 @@ bool use_chunk(const GemmProblem* q, int n, int esize, bool fp32_operands, int s
 // often, a smaller one starts more waves.  MI355X, k-chunk kernel, fp32 storage,
 // 16-bit operands, us for 16 / 32 / 64: 512 x 512 x 2000 split 2 (256 large tiles)
 // 29.7 / 23.2 / 16.6, 512 x 784 x 256 (32 large, 128 middle tiles) 8.9 / 11.1
-// / 17.6, 1024^3 54 / 41 / 19.7.
+// / 17.6, 1024^3 54 / 41 / 19.7.  Tile kernel: 64 x 64 from 64 of them on, over all
+// problems of a launch, also where fewer than 64 rows or columns leave them half
+// empty ((10, 4096 x 3, 784) nets at B = 32, fp16, split 2: prediction phase 378 us
+// on 32 x 32, 295 on 64 x 64, inference 298, 234; (10, 4096 x 2, 784) at B = 20 491,
+// 292; nine more nets of 300-20,000 wide layers and B = 17-4096 the same either way).
 int pick_tile(int tile, const GemmProblem* q, int n, bool chunk) {
   const long long t64 = count_tiles(q, n, 64);
   if (chunk) {
