@@ -193,8 +193,11 @@ typedef struct ipc_plan ipc_plan;
  *                    storage, every output width d_0..d_{L-1} <= 128, L <= 16,
  *                    split 1 or 3, one column block's buffers fit in LDS), the
  *                    column-block whole-step kernel for widths <= 64 and B <=
- *                    128 and the phased path beyond; else the wide GEMM path
- *                    when eligible, else the phased path;
+ *                    128, and for a few small nets beyond (two weights of at
+ *                    most 96 x 128 at B <= 64; IPC_WMODE_OUTER at B > 17 with
+ *                    every d_1..d_L <= 512 and widths <= 96 or L <= 3), the
+ *                    phased path for the others; else the wide GEMM path when
+ *                    eligible, else the phased path;
  *   IPC_PATH_PHASED  one generic multi-layer launch per phase (any config);
  *   IPC_PATH_NARROW  the column-block whole-step kernel (IPC_ERR_CONFIG if
  *                    not narrow);

@@ -905,16 +905,28 @@ bool narrow_outer(int B, int wmode) {
 // Whether an automatic plan leaves a narrow net to the phased path's k-chunk
 // launches.  The column kernel's 16-column blocks re-read every W in a few
 // workgroups, phase after phase; the k-chunk kernel spreads the same products,
-// added in the same order, over the chip and is ahead at every measured size
-// (MI355X, us, initialisation / 4 steps, column kernel -> k-chunk launches:
-// 784 x 128^4 fp16 at B = 20, 128, 512, 1024 35 / 200 -> 21 / 72, 35 / 197 ->
-// 21 / 75, 35 / 247 -> 21 / 116, 36 / 349 -> 25 / 158; 784 x 128^2 fp32 at B =
-// 16 25 / 124 -> 14 / 68; 784 x 64^2 at B = 256 24 / 144 -> 17 / 75).  The
-// sizes the layer-resident kernel is laid out for (widths <= 64, B <= 128) keep
-// a whole-step kernel also where that one does not fit, so that a plan and
-// ipc_steps_noalloc, which only has those, agree there bit for bit.
-bool column_is_slow(int L, const int* dims, int B) {
-  return B > RES_MAX_B || *std::max_element(dims, dims + L) > RES_MAX_WIDTH;
+// added in the same order, over the chip (MI355X, us, initialisation / 4 steps,
+// column kernel -> k-chunk launches: 784 x 128^4 fp16 at B = 20, 128, 512, 1024 35 /
+// 200 -> 21 / 72, 35 / 197 -> 21 / 75, 35 / 247 -> 21 / 116, 36 / 349 -> 25 / 158; 784 x
+// 128^2 fp32 at B = 16 25 / 124 -> 14 / 68; 784 x 64^2 at B = 256 24 / 144 -> 17 / 75;
+// 784 x 64^3 fp32 at B = 2048 34 / 671 -> 27 / 136, 65536 501 / 38,858 -> 226 / 2,595;
+// 784 x 128^3 fp32 at B = 4096 46 / 2,125 -> 44 / 463, 65536 634 / 34,448 -> 383 /
+// 5,880).  Not where the launches are too many for what they do:
+// * two weights of at most 96 x 128, B <= 64 ((3, 66, 20) fp32, rank-B update, B = 4,
+//   4 steps 51 / 63; (10, 65, 64) 58 / 65; at B = 128 64 / 63);
+// * the rank-B update, a launch a layer, past B = 17, where the column kernel runs
+//   a GEMM instead, for short contractions and narrow or few layers ((10, 65 x 4,
+//   256) fp32, B = 32, 135 / 156, (10, 65 x 2, 400) 110 / 119, 550 156 / 122; (10,
+//   128 x 2, 256) 118 / 122, (10, 128 x 4, 256) 190 / 159; at B = 16 and 17 the
+//   launches are level or ahead).
+// The sizes the layer-resident kernel is laid out for (widths <= 64, B <= 128) keep
+// a whole-step kernel also where that one does not fit.
+bool column_is_slow(int L, const int* dims, int B, int wmode) {
+  const int width = *std::max_element(dims, dims + L), kmax = *std::max_element(dims + 1, dims + L + 1);
+  if (B <= RES_MAX_B && width <= RES_MAX_WIDTH) return false;
+  if (B <= 64 && L == 2 && width <= 96 && kmax <= 128) return false;
+  if (wmode == IPC_WMODE_OUTER && B > 17 && kmax <= 512 && (width <= 96 || L <= 3)) return false;
+  return true;
 }
 
 // Layer-resident kernel eligibility; fills `ra` and returns its workspace bytes, or -1.
@@ -1091,7 +1103,8 @@ int ipc_plan_create(ipc_plan** out, int L, const int* dims, int B, int storage, 
     }
   }
   int narrow_cap = 256;
-  if (eligible && ((path == IPC_PATH_AUTO && !column_is_slow(L, dims, B)) || path == IPC_PATH_NARROW || path == IPC_PATH_RESIDENT)) {
+  const bool column = eligible && !column_is_slow(L, dims, B, weight_mode);
+  if ((path == IPC_PATH_AUTO && column) || (eligible && (path == IPC_PATH_NARROW || path == IPC_PATH_RESIDENT))) {
     const int lds = narrow_lds_bytes(dims, L, operand, esplit);
     const int cap = coresident_capacity([&] { return narrow_prepare(operand, esplit, act, lds); },
                                         [&](int* n) { return narrow_occupancy(operand, esplit, act, lds, n); });
@@ -1116,7 +1129,6 @@ int ipc_plan_create(ipc_plan** out, int L, const int* dims, int B, int storage, 
   p->spin_limit = kNarrowSpinLimit;
   p->narrow_cap = narrow_cap;
   p->resident = path == IPC_PATH_RESIDENT || (path == IPC_PATH_AUTO && res_bytes >= 0);
-  const bool column = eligible && !column_is_slow(L, dims, B);
   p->narrow = p->resident || path == IPC_PATH_NARROW || (path == IPC_PATH_AUTO && column);
   p->wide = !p->narrow && (path == IPC_PATH_WIDE || (path == IPC_PATH_AUTO && weligible && !eligible));
   if (p->narrow) p->ws_bytes = narrow_workspace_bytes(dims, L, B, p->recompute != 0);

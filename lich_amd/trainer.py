@@ -89,8 +89,8 @@ class IPCConfig:
     resident_rows: int | None = None
     # Kernel path: "auto" (the layer-resident whole-step kernel when eligible,
     # else for narrow nets the column-block whole-step kernel up to width 64 and
-    # B = 128 and phased beyond, else the wide GEMM path when eligible, else
-    # phased), "resident", "narrow" / "on",
+    # B = 128 and for a few small nets beyond, phased for the others, else the
+    # wide GEMM path when eligible, else phased), "resident", "narrow" / "on",
     # "wide", "phased" / "off".
     fused: str = "auto"
 

@@ -69,3 +69,28 @@ def test_generic_tiles_run_as_asked_for(kind, M, K, B):
 def test_many_tiles_of_a_partly_filled_round(kind, M, K, B, st, act, chunk):
     """Loaders with a costly activation: the tile kernel, which the k-chunk kernel had slowed down."""
     assert (route(kind, M, K, B, st=st, act=act) in CHUNK) == chunk
+
+
+@pytest.mark.parametrize("dims,B,wmode,op,want", [
+    # the rank-B update, a launch a layer on the phased path
+    ((10, 65, 65, 65, 65, 256), 32, "outer", "fp32", "narrow"), ((10, 65, 65, 65, 65, 256), 17, "outer", "fp32", "phased"),
+    ((10, 65, 65, 550), 32, "outer", "fp32", "phased"), ((10, 128, 128, 256), 24, "outer", "fp16", "narrow"),
+    ((10, 128, 128, 128, 128, 256), 24, "outer", "fp16", "phased"), ((10, 65, 65, 256), 32, "gemm", "fp32", "phased"),
+    # a few small layers
+    ((3, 66, 20), 4, "auto", "fp32", "narrow"), ((10, 65, 64), 64, "gemm", "fp16", "narrow"),
+    ((10, 65, 64), 65, "gemm", "fp16", "phased"), ((10, 65, 129), 64, "gemm", "fp16", "phased"),
+    ((10, 128, 64), 4, "gemm", "fp32", "phased"), ((10, 65, 65, 64), 4, "gemm", "fp32", "phased"),
+    # no upper end in B
+    ((10, 64, 64, 64, 784), 65536, "gemm", "fp32", "phased"),
+])
+def test_automatic_path_of_narrow_nets_past_the_resident_sizes(dims, B, wmode, op, want):
+    import ctypes
+
+    lib, h = nat.lib(), ctypes.c_void_p()
+    code = {"fp32": nat.DT_F32, "fp16": nat.DT_F16}[op]
+    assert lib.ipc_plan_create(ctypes.byref(h), len(dims) - 1, (ctypes.c_int * len(dims))(*dims), B, 0, code, 1,
+                               nat.act_code("tanh"), 1e-4, 0.5, 1, nat.WMODE[wmode], nat.FUSED["auto"]) == nat.IPC_OK
+    try:
+        assert nat.PATH_NAMES[lib.ipc_plan_path(h)] == want
+    finally:
+        lib.ipc_plan_destroy(h)
