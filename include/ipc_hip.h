@@ -379,14 +379,13 @@ int ipc_plan_graph_steps(const ipc_plan* plan);
  * No counterpart in the reference: an entry point for callers that cannot
  * allocate device memory (code under hipGraph capture, tight serving loops,
  * harnesses that forbid hipMalloc).  Runs `steps` iPC steps of a narrow net
- * on the whole-step kernels exactly as a plan created with IPC_PATH_AUTO
- * (widths above 64 or B above 128: IPC_PATH_NARROW), fp32 storage and
- * recompute mode would (ipc_plan_create + ipc_plan_bind + ipc_plan_step: same
- * kernels, same results), without a plan or a caller
- * workspace: the kernels' barrier words, f(x) buffers and exchange records
- * live in the library's static device scratch, 8 MiB per GPU, held until the
- * process ends.  A net that needs more is refused with IPC_ERR_SHAPE; one the
- * whole-step kernels do not take (a width above 128, L above 16, split 2)
+ * exactly as a plan created with IPC_PATH_AUTO, fp32 storage and recompute
+ * mode would (ipc_plan_create + ipc_plan_bind + ipc_plan_step: same kernels,
+ * same results), without a plan or a caller workspace: the whole-step kernels'
+ * barrier words, f(x) buffers and exchange records live in the library's static
+ * device scratch, 8 MiB per GPU, held until the process ends.  A net whose
+ * whole-step kernels would need more is refused with IPC_ERR_SHAPE; one they
+ * do not take (a width above 128, L above 16, split 2)
  * with IPC_ERR_CONFIG.  x (L+1 pointers), e (L pointers, e[L] unused) and w
  * (L pointers) are laid out as for ipc_plan_bind; the caller does the forward
  * initialisation.  Each call clears the scratch words that must start at

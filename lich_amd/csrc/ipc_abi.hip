@@ -942,24 +942,72 @@ long long resident_eligible(int L, const int* dims, int B, int operand, int spli
   return resident_plan(dims, L, B, split == IPC_SPLIT_WX ? 3 : 1, 2, false, top_rows, ra);
 }
 
-// Kernels and tiles of the phased launches (tiles as set by ipc_plan_set_tiles
-// or automatic; with 16-bit storage a tile set by id is the tile kernel's, as in
-// the standalone calls).  A net that the wide path could run as well keeps the tile
-// kernel: its k order is the wide path's, so the two paths' 16-bit operands
-// round alike and their states agree to fp32 rounding over many steps.
+// Whether the phased path runs the rank-B weight update, a launch a layer.
+bool rank_b_launches(int B, int wmode) {
+  return wmode == IPC_WMODE_OUTER || (wmode == IPC_WMODE_AUTO && B <= 16);
+}
+
+// The problems of one phased step: L predictions, L - 1 inference updates and L
+// weight updates, in `outer` or `weight`.  `a`: the saved activations, NULL in
+// recompute mode.
+void phase_problems(int L, const int* d, int B, void* const* x, void* const* e, void* const* w, void* const* a,
+                    float alpha, float gamma, bool rank_b, int act, int es, GemmProblem* pred, GemmProblem* infer,
+                    GemmProblem* weight, OuterProblem* outer) {
+  for (int l = 0; l < L; ++l) {
+    // Prediction always applies f to x[l+1] in its loader (trainer.py:617-618);
+    // only the weight update consumes the saved activation.
+    pred[l] = make_pf(KIND_PRED, x[l + 1], w[l], x[l], e[l], d[l], d[l + 1], B, 1, act, es);
+    if (l > 0)
+      infer[l - 1] = make_inf(x[l], e[l], w[l - 1], e[l - 1], a ? a[l] : nullptr, d[l], d[l - 1], B, 1, gamma, act, es);
+    const void* src = a ? a[l + 1] : x[l + 1];
+    if (rank_b) outer[l] = make_outer(w[l], e[l], src, d[l], d[l + 1], B, 1, alpha, !a, act);
+    else weight[l] = make_wgt(w[l], e[l], src, d[l], d[l + 1], B, 1, alpha, !a, act, es);
+  }
+}
+
+// Kernel and tile of a phased launch (`want`: a tile set by ipc_plan_set_tiles or
+// automatic; with 16-bit storage a tile set by id is the tile kernel's, as in the
+// standalone calls).  `chain`: a net that the wide path could run as well keeps
+// the tile kernel: its k order is the wide path's, so the two paths' 16-bit
+// operands round alike and their states agree to fp32 rounding over many steps.
+int phase_tile(int want, const GemmProblem* v, int n, int storage, int operand, int split, bool chain) {
+  const int es = elem_size(storage);
+  const bool chunk = !chain && (es == 4 || want == IPC_TILE_AUTO) &&
+                     use_chunk(v, n, es, operand == IPC_DT_F32, n > 0 && v[0].kind == KIND_PRED ? split : IPC_SPLIT_NONE);
+  return pick_tile(want, v, n, chunk);
+}
+
 void pick_phase_tiles(ipc_plan* plan) {
   const bool chain = wide_eligible(plan->storage, plan->operand, plan->split, plan->wmode, plan->B) &&
                      !narrow_eligible(plan->L, plan->dims.data(), plan->storage, plan->operand, plan->split);
-  const int es = elem_size(plan->storage), *t = plan->tile_override;
-  auto pick = [&](int want, const std::vector<GemmProblem>& v) {
-    const int split = v.empty() || v[0].kind != KIND_PRED ? IPC_SPLIT_NONE : plan->split;
-    const bool chunk = !chain && (es == 4 || want == IPC_TILE_AUTO) &&
-                       use_chunk(v.data(), (int)v.size(), es, plan->operand == IPC_DT_F32, split);
-    return pick_tile(want, v.data(), (int)v.size(), chunk);
+  auto pick = [&](int phase, const std::vector<GemmProblem>& v) {
+    return phase_tile(plan->tile_override[phase], v.data(), (int)v.size(), plan->storage, plan->operand, plan->split, chain);
   };
-  plan->tile_pred = pick(t[0], plan->pred);
-  plan->tile_infer = pick(t[1], plan->infer);
-  plan->tile_weight = pick(t[2], plan->weight);
+  plan->tile_pred = pick(0, plan->pred);
+  plan->tile_infer = pick(1, plan->infer);
+  plan->tile_weight = pick(2, plan->weight);
+}
+
+// `steps` steps of a narrow net on the phased path's launches without a plan: fp32
+// storage, recompute mode, as an automatic plan runs them.
+int phased_steps(int L, const int* d, int B, void* const* x, void* const* e, void* const* w, int operand, int split,
+                 int act, float alpha, float gamma, int wmode, int steps, hipStream_t s) {
+  GemmProblem pred[NARROW_MAX_L], infer[NARROW_MAX_L], weight[NARROW_MAX_L];
+  OuterProblem outer[NARROW_MAX_L];
+  const bool rank_b = rank_b_launches(B, wmode);
+  phase_problems(L, d, B, x, e, w, nullptr, alpha, gamma, rank_b, act, 4, pred, infer, weight, outer);
+  auto tile = [&](const GemmProblem* v, int n) { return phase_tile(IPC_TILE_AUTO, v, n, IPC_DT_F32, operand, split, false); };
+  const int tp = tile(pred, L), ti = tile(infer, L - 1), tw = rank_b ? 0 : tile(weight, L);
+  for (int t = 0; t < steps; ++t) {
+    TRY(launch_rc(launch_gemm(pred, L, IPC_DT_F32, operand, split, tp, s), "prediction phase"));
+    if (L > 1) TRY(launch_rc(launch_gemm(infer, L - 1, IPC_DT_F32, operand, IPC_SPLIT_NONE, ti, s), "inference phase"));
+    if (rank_b) {
+      for (int l = 0; l < L; ++l) TRY(launch_rc(launch_outer(outer[l], IPC_DT_F32, s), "outer weight update"));
+    } else {
+      TRY(launch_rc(launch_gemm(weight, L, IPC_DT_F32, operand, IPC_SPLIT_NONE, tw, s), "weight phase"));
+    }
+  }
+  return ok();
 }
 
 int launch_narrow_mode(ipc_plan* plan, int mode, int steps, hipStream_t s) {
@@ -1185,22 +1233,12 @@ int ipc_plan_bind(ipc_plan* plan, void* const* x, void* const* e, void* const* w
   }
   const std::vector<int>& d = plan->dims;
   plan->pred.clear(); plan->infer.clear(); plan->weight.clear(); plan->outer.clear(); plan->fwd.clear();
-  // Prediction always applies f to x[l+1] in its loader (trainer.py:617-618);
-  // only the weight update consumes the saved activation.
-  for (int l = 0; l < L; ++l)
-    plan->pred.push_back(make_pf(KIND_PRED, x[l + 1], w[l], x[l], e[l], d[l], d[l + 1], B, 1, plan->act, es));
-  for (int l = 1; l < L; ++l) {
-    plan->infer.push_back(make_inf(x[l], e[l], w[l - 1], e[l - 1], plan->recompute ? nullptr : a[l], d[l],
-                                   d[l - 1], B, 1, plan->gamma, plan->act, es));
-  }
-  for (int l = 0; l < L; ++l) {
-    const bool use_outer = plan->wmode == IPC_WMODE_OUTER || (plan->wmode == IPC_WMODE_AUTO && B <= 16);
-    const void* src = plan->recompute ? x[l + 1] : a[l + 1];
-    if (use_outer)
-      plan->outer.push_back(make_outer(w[l], e[l], src, d[l], d[l + 1], B, 1, plan->alpha, plan->recompute, plan->act));
-    else
-      plan->weight.push_back(make_wgt(w[l], e[l], src, d[l], d[l + 1], B, 1, plan->alpha, plan->recompute, plan->act, es));
-  }
+  const bool outer = rank_b_launches(B, plan->wmode);
+  plan->pred.resize(L);
+  plan->infer.resize(L - 1);
+  (outer ? plan->outer.resize(L) : plan->weight.resize(L));
+  phase_problems(L, d.data(), B, x, e, w, plan->recompute ? nullptr : a, plan->alpha, plan->gamma, outer, plan->act, es,
+                 plan->pred.data(), plan->infer.data(), plan->weight.data(), plan->outer.data());
   plan->act_src = x[L];
   plan->act_dst = plan->recompute ? nullptr : a[L];
   for (int l = L - 1; l >= 1; --l)
@@ -1663,6 +1701,8 @@ int ipc_steps_noalloc(int L, const int* dims, int B, void* const* x, void* const
                 "this net needs %lld bytes of scratch; the library's static scratch holds %lld (use a plan with a "
                 "caller workspace)", need, kScratchBytes);
   if (steps == 0) return ok();
+  if (column_is_slow(L, dims, B, weight_mode))
+    return phased_steps(L, dims, B, x, e, w, operand, esplit, act, alpha, gamma, weight_mode, steps, (hipStream_t)stream);
   char* ws = nullptr;
   TRY(scratch_address(&ws));
   if (res_bytes >= 0) {
