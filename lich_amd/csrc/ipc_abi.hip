@@ -115,6 +115,10 @@ bool chunk_fits(const GemmProblem& q, int esize) {
   return ((a_rows + 64) * q.lda + 64) * esize < (1LL << 31) && ((b_rows + 64) * q.ldb + 64) * esize < (1LL << 31);
 }
 
+// Threads of a launch stay below this (workgroups of the k-chunk kernel: up to
+// 512, and 1024 on its 16 x 16 tiles, which few tiles take only).
+constexpr long long kMaxThreads = 1LL << 32;
+
 // Output tiles of edge `e` over `n` problems.
 long long count_tiles(const GemmProblem* q, int n, int e) {
   long long t = 0;
@@ -152,6 +156,7 @@ bool use_chunk(const GemmProblem* q, int n, int esize, bool fp32_operands, int s
   if (n == 0) return true;
   const bool infer = q[0].kind == KIND_INFER;
   const long long t64 = count_tiles(q, n, 64);
+  if (t64 * 512 >= kMaxThreads) return false;
   if (t64 > 256 && kmax <= 128) return false;
   if (t64 > 512 && kmax <= (infer ? 256 : 512)) return false;
   if (n == 1 && !infer && t64 >= (split == IPC_SPLIT_WX ? 2048 : 1024) && kmax <= 1408) {
@@ -180,7 +185,8 @@ bool use_chunk(const GemmProblem* q, int n, int esize, bool fp32_operands, int s
 int pick_tile(int tile, const GemmProblem* q, int n, bool chunk) {
   const long long t64 = count_tiles(q, n, 64);
   if (chunk) {
-    if (tile != IPC_TILE_AUTO) return tile == IPC_TILE_32x32 ? TILE_CHUNK_32 : TILE_CHUNK_64;
+    const bool t32 = tile == IPC_TILE_32x32 && count_tiles(q, n, 32) * 512 < kMaxThreads;
+    if (tile != IPC_TILE_AUTO) return t32 ? TILE_CHUNK_32 : TILE_CHUNK_64;
     return t64 >= 192 ? TILE_CHUNK_64 : count_tiles(q, n, 32) >= 256 ? TILE_CHUNK_32 : TILE_CHUNK_16;
   }
   if (tile != IPC_TILE_AUTO) return tile;

@@ -94,3 +94,13 @@ def test_automatic_path_of_narrow_nets_past_the_resident_sizes(dims, B, wmode, o
         assert nat.PATH_NAMES[lib.ipc_plan_path(h)] == want
     finally:
         lib.ipc_plan_destroy(h)
+
+
+def test_launches_stay_below_the_thread_limit():
+    """2^23 groups of one tile: 2^32 threads in the k-chunk kernel's workgroups of
+    512, which a launch may not have; the tile kernel's 256 fit, as before it."""
+    assert route(INFER, 16, 257, 16, groups=(1 << 23) - 1) == 18
+    assert route(INFER, 16, 257, 16, groups=1 << 23) == 2
+    assert route(INFER, 16, 257, 16, groups=1 << 23, st="fp32") == 2
+    assert route(INFER, 128, 257, 128, groups=1 << 18, st="fp32", tile=0) == 17
+    assert route(INFER, 128, 257, 128, groups=1 << 19, st="fp32", tile=0) == 18  # 2^23 tiles of 32 x 32
