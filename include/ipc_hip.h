@@ -60,12 +60,13 @@ extern "C" {
 #define IPC_ACT_GELU 5
 
 /* tile configurations of the MFMA GEMM family; IPC_TILE_AUTO picks by shape.
- * The generic ids 0-2 name 32 x 32, 64 x 64 and 128 x 128 output tiles.  With
- * fp32 storage they run on the k-chunk kernel (the contraction split over a
- * workgroup's waves; 128 x 128 names its largest tile, 64 x 64) wherever that is
- * the faster one, else on the tile kernel; the bits depend on the kernel, not on
- * the tile.  With 16-bit storage the ids name the tile kernel, whose k order is
- * the LDS-DMA kernel's.  IPC_TILE_AUTO also picks the k-chunk kernel's 16 x 16.
+ * The generic ids 0-2 name 32 x 32, 64 x 64 and 128 x 128 output tiles on the
+ * tile kernel.  With fp32 storage they run on the k-chunk kernel (the contraction
+ * split over a workgroup's waves) wherever that is the faster one, as 32 x 32
+ * (16 x 16 where there are fewer than 256 of them), 64 x 64 (32 x 32 where fewer
+ * than 192) and 64 x 64; the bits depend on the kernel, not on the tile.  With
+ * 16-bit storage the ids name the tile kernel, whose k order is the LDS-DMA
+ * kernel's.
  * IPC_TILE_DMA_* are the LDS-DMA kernel (operands streamed HBM -> LDS without
  * VGPR staging, transposed operands read with the LDS transpose read) in
  * four tile configurations: 256 x 128, 128 x 256,
@@ -84,8 +85,8 @@ extern "C" {
  * operands are below 2^31 bytes each go to the generic kernels instead: the
  * k-chunk kernel, or the tile kernel for inference updates of more than 256
  * such tiles and a contraction of at most 128.  Asking for a DMA tile
- * where they do not hold is IPC_ERR_CONFIG.  The autotuner
- * searches all of them per shape. */
+ * where they do not hold is IPC_ERR_CONFIG.  The autotuner times the automatic
+ * choice and every id per shape. */
 #define IPC_TILE_AUTO (-1)
 #define IPC_TILE_32x32 0
 #define IPC_TILE_64x64 1
@@ -301,11 +302,13 @@ int ipc_plan_set_tiles(ipc_plan* plan, int tile_pred, int tile_infer, int tile_w
  * IPC_PATH_WIDE plans, the counterpart of the reference's per-shape
  * KernelConfig search, scripts/autotune.py:51-131).  ipc_plan_wide_config_count
  * gives the configurations a phase offers (IPC_PHASE_PRED with split
- * IPC_SPLIT_NONE or IPC_SPLIT_W, IPC_PHASE_INFER, IPC_PHASE_WEIGHT); 0 is the
- * default, and every configuration of a phase gives bit-identical results.
- * ipc_plan_set_wide_config selects one per phase (-1 = default) and the
- * number of k-slices of the output layer's prediction (-1 = chosen at bind
- * from the device's CU count; 1 = none; else a power of two up to 16).  It is
+ * IPC_SPLIT_NONE or IPC_SPLIT_W, IPC_PHASE_INFER, IPC_PHASE_WEIGHT); every one
+ * of a phase gives bit-identical results.  ipc_plan_set_wide_config selects one
+ * per phase (-1, the default = chosen at bind for the shortest estimated launch,
+ * among them 64 x 64 tiles that have no id) and the number of k-slices of the
+ * output layer's prediction (-1 = chosen at bind from the device's CU count and
+ * the tiles of the configuration asked for, 0 where none is; 1 = none; else a
+ * power of two up to 16).  It is
  * called after ipc_plan_create and before ipc_plan_workspace_bytes /
  * ipc_plan_bind (the prediction tile sets the workspace size); a k-split the
  * net cannot take fails at bind with IPC_ERR_CONFIG. */

@@ -170,9 +170,15 @@ bool use_chunk(const GemmProblem* q, int n, int esize, bool fp32_operands, int s
   return !(esize == 4 && !infer && kmax >= 1024 && count_tiles(q, n, 128) >= 512);
 }
 
-// Tile of such a launch.  `tile`: IPC_TILE_AUTO, or a generic tile id, which
-// names 32 x 32, 64 x 64 or 128 x 128 tiles; the k-chunk kernel's largest is 64 x 64
-// (neither kernel's bits depend on the tile).  Automatic: the largest tile that
+// Tile of such a launch.  `tile`: IPC_TILE_AUTO, or a generic tile id: 32 x 32,
+// 64 x 64 or 128 x 128 on the tile kernel.  On the k-chunk kernel 32 x 32 (16 x 16
+// where there are fewer than 256 of them), 64 x 64 (32 x 32 where fewer than 192)
+// and 64 x 64: no id runs a larger tile than it names and each automatic choice
+// has an id (4096 x 4096 x 2048 inference, ids 0 / 1 / 2, tile kernel 789 / 567 / 617
+// us, these 547 / 270 / 270, 16 x 16 tiles 2,126; of 38 shapes two are slower by a
+// named tile: inference 8192 x 300 x 2048 id 1 103 / 136, weight update 2048 x 2048, B =
+// 2048, 128 / 136).
+// Neither kernel's bits depend on the tile.  Automatic: the largest tile that
 // gives the 256 CUs about a workgroup each; a larger tile reads its operands less
 // often, a smaller one starts more waves.  MI355X, k-chunk kernel, fp32 storage,
 // 16-bit operands, us for 16 / 32 / 64: 512 x 512 x 2000 split 2 (256 large tiles)
@@ -185,9 +191,11 @@ bool use_chunk(const GemmProblem* q, int n, int esize, bool fp32_operands, int s
 int pick_tile(int tile, const GemmProblem* q, int n, bool chunk) {
   const long long t64 = count_tiles(q, n, 64);
   if (chunk) {
-    const bool t32 = tile == IPC_TILE_32x32 && count_tiles(q, n, 32) * 512 < kMaxThreads;
-    if (tile != IPC_TILE_AUTO) return t32 ? TILE_CHUNK_32 : TILE_CHUNK_64;
-    return t64 >= 192 ? TILE_CHUNK_64 : count_tiles(q, n, 32) >= 256 ? TILE_CHUNK_32 : TILE_CHUNK_16;
+    const long long t32 = count_tiles(q, n, 32);
+    if (tile == IPC_TILE_32x32) return t32 * 512 >= kMaxThreads ? TILE_CHUNK_64 : t32 >= 256 ? TILE_CHUNK_32 : TILE_CHUNK_16;
+    if (tile == IPC_TILE_64x64) return t64 >= 192 ? TILE_CHUNK_64 : TILE_CHUNK_32;
+    if (tile == IPC_TILE_128x128) return TILE_CHUNK_64;
+    return t64 >= 192 ? TILE_CHUNK_64 : t32 >= 256 ? TILE_CHUNK_32 : TILE_CHUNK_16;
   }
   if (tile != IPC_TILE_AUTO) return tile;
   return count_tiles(q, n, 128) >= 512 ? IPC_TILE_128x128 : t64 >= 64 ? IPC_TILE_64x64 : IPC_TILE_32x32;

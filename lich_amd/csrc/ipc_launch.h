@@ -65,7 +65,7 @@ hipError_t launch_outer(const OuterProblem& p, int storage, hipStream_t s);
 hipError_t launch_act(const void* src, void* dst, long long n, int act, int storage, hipStream_t s);
 
 // Tile ids of the k-chunk kernel (ipc_chunk_kernel.h), next to the tile
-// kernel's 0-2.
+// kernel's 0-2; the ABI's generic tile ids 0-2 map to them in order.
 enum { TILE_CHUNK_16 = 16, TILE_CHUNK_32 = 17, TILE_CHUNK_64 = 18 };
 hipError_t launch_chunk_pf(const GemmProblem* probs, int count, int storage, int operand, int split, int tile,
                            hipStream_t s);

@@ -35,10 +35,10 @@ class KernelConfig:
     """Tile configuration (reference ``tilelang_kernels.py:8-17``).
 
     ``tile`` selects one of the CDNA4 MFMA tile shapes of the library
-    (generic kernels 0: 32x32, 1: 64x64, 2: 128x128, which the k-chunk kernel
-    of fp32 storage runs as 64x64; LDS-DMA kernel for 16-bit storage 3:
-    256x128, 4: 128x256, 5: 128x128, 6: 256x256; -1: kernel and tile chosen
-    from the problem shape).  When
+    (generic kernels 0: 32x32, 1: 64x64, 2: 128x128, on the k-chunk kernel of
+    fp32 storage 64x64 at most and smaller where there are few; LDS-DMA kernel
+    for 16-bit storage 3: 256x128, 4: 128x256, 5: 128x128, 6: 256x256; -1:
+    kernel and tile chosen from the problem shape).  When
     ``tile`` is None the reference's ``block_m``/``block_n`` pick the closest
     shape; with neither given the choice is automatic.
     """

@@ -50,12 +50,15 @@ def test_workspace_bytes_are_those_of_the_call():
         lib.ipc_set_s16_preactivate(-1)
 
 
-@pytest.mark.parametrize("kind", [PRED, INFER, WEIGHT])
-@pytest.mark.parametrize("M,K,B", [(64, 784, 128), (512, 784, 256), (512, 512, 2000), (1024, 1024, 1024)])
-def test_generic_tiles_run_as_asked_for(kind, M, K, B):
-    assert [route(kind, M, K, B, st="fp32", tile=t) for t in (0, 1, 2)] == [17, 18, 18]  # k-chunk: 64 x 64 at most
-    assert [route(kind, M, K, B, st="fp16", tile=t) for t in (0, 1, 2)] == [0, 1, 2]     # the tile kernel
-    assert route(kind, 4096, 4096, 2048, st="fp32", tile=0) == (17 if kind == INFER else 0)
+@pytest.mark.parametrize("M,N,want", [(64, 128, [16, 17, 18]), (512, 480, [16, 17, 18]), (512, 512, [17, 17, 18]),
+                                      (704, 1088, [17, 17, 18]), (768, 1024, [17, 18, 18]), (1024, 1024, [17, 18, 18])])
+def test_generic_tiles_run_as_asked_for(M, N, want):
+    """No id runs a larger tile than it names, and each automatic choice has an id."""
+    for call in ((PRED, M, 300, N), (INFER, M, 300, N), (WEIGHT, M, N, 300)):
+        ids = [route(*call, st="fp32", tile=t) for t in (0, 1, 2)]
+        assert ids == want and route(*call, st="fp32") in ids
+        assert [route(*call, st="fp16", tile=t) for t in (0, 1, 2)] == [0, 1, 2]  # the tile kernel
+    assert route(PRED, 4096, 4096, 2048, st="fp32", tile=0) == 0 and route(INFER, 4096, 4096, 2048, st="fp32", tile=0) == 17
 
 
 @pytest.mark.parametrize("kind,M,K,B,st,act,chunk", [
@@ -102,5 +105,4 @@ def test_launches_stay_below_the_thread_limit():
     assert route(INFER, 16, 257, 16, groups=(1 << 23) - 1) == 18
     assert route(INFER, 16, 257, 16, groups=1 << 23) == 2
     assert route(INFER, 16, 257, 16, groups=1 << 23, st="fp32") == 2
-    assert route(INFER, 128, 257, 128, groups=1 << 18, st="fp32", tile=0) == 17
-    assert route(INFER, 128, 257, 128, groups=1 << 19, st="fp32", tile=0) == 18  # 2^23 tiles of 32 x 32
+    assert [route(INFER, 128, 257, 128, groups=g, st="fp32", tile=0) for g in (1 << 18, 1 << 19)] == [17, 18]
