@@ -3,15 +3,16 @@ search and ``scripts/hierarchical_autotune.py`` execution search, reduced to
 this library's choices), every candidate gated on correctness.
 
 * Kernel level: for every prediction / inference / weight shape of the net,
-  each tile configuration of the standalone kernels (generic 32x32, 64x64,
-  128x128 and the LDS-DMA tile) is run on seeded data, checked against torch
+  each tile configuration of the standalone kernels (the generic and the LDS-DMA
+  tiles; with 16-bit storage also the automatic choice) is run on seeded data,
+  checked against torch
   on the device with the reference's probe (``autotune.py:250-260``: at most
   1 % of the elements outside ``atol + rtol |ref|``, rtol = atol = 2e-2) and,
   if it passes, timed (HIP events around graph replays of back-to-back
   launches, the method of ``autotune.py:200-215``); the fastest passing one
   goes into a TuningTable (schema 1).
-* Wide path (nets the wide GEMM path serves): each phase's tile
-  configurations and the k-split of the output layer's prediction
+* Wide path (nets the wide GEMM path serves): the automatic choice and each
+  phase's tile configurations and the k-split of the output layer's prediction
   (``ipc_plan_set_wide_config``).  A candidate runs one step from a fixed
   state, is checked against a float32 torch step on the device with the same
   probe (states, errors, weight deltas), and its phase launch is then timed;
@@ -24,9 +25,9 @@ this library's choices), every candidate gated on correctness.
   choices through the reference's precedence.
 
 * Standalone kernels with 16-bit storage (the per-kernel sweep's operator
-  calls, ``tune_standalone``): the generic tiles and the four LDS-DMA tile
-  configurations (256x128, 128x256, 128x128, 256x256) per (kind, M, K, B), under the
-  same probe.
+  calls, ``tune_standalone``): the automatic choice, the generic tiles and the
+  four LDS-DMA tile configurations (256x128, 128x256, 128x128, 256x256) per (kind,
+  M, K, B), under the same probe.
 * Layer-resident plans: the top layer's row-block size (16, 32 or 64 rows,
   ``ipc_plan_set_resident_rows``) is part of the execution search; every
   execution candidate runs one step from the forward-initialised state and
@@ -34,7 +35,9 @@ this library's choices), every candidate gated on correctness.
   torch step before it is timed.
 
 Candidates that fail the probe are never selected; they are recorded with
-the reason (``rejected``).
+the reason (``rejected``).  A named choice is kept only where it beats the
+automatic one by ``AUTO_MARGIN``, so that a tuned net is not slower than an
+untuned one.
 
     python -m lich_amd.autotune --dims 10,64,64,64,784 --batch 128 --activation tanh \\
         --dtype float16 --table results/tuning_cdna4.json --policy results/hierarchical_policy.json
@@ -56,8 +59,12 @@ from .reference import get_activation
 from .trainer import HipIPC, IPCConfig, init_weights_cpu
 from .tuning import TuningEntry, TuningKey, TuningTable, config_to_dict
 
-TILES = (0, 1, 2, 3, 4, 5, 6)  # generic 32x32, 64x64, 128x128; LDS-DMA 256x128, 128x256, 128x128, 256x256
+# automatic (16-bit storage: the only way to the k-chunk kernel and to the LDS-DMA kernel's 512x64; with fp32
+# storage every automatic choice has an id); generic small, middle, large; LDS-DMA 256x128, 128x256, 128x128, 256x256
+TILES = (-1, 0, 1, 2, 3, 4, 5, 6)
 RESIDENT_ROWS = (16, 32, 64)
+# a named choice replaces the automatic one when it is this much faster (two runs of one choice differ by about 1 %)
+AUTO_MARGIN = 0.98
 RTOL = ATOL = 2e-2
 MAX_BAD = 0.01
 
@@ -153,7 +160,7 @@ def tune_kernels(dims, B: int, activation: str, dtype: torch.dtype, *, reps: int
     entries = []
     for kind, M, K in (shapes if shapes is not None else net_shapes([int(d) for d in dims])):
         best = None
-        for tile in TILES:
+        for tile in TILES[1:] if storage == torch.float32 else TILES:
             cfg = KernelConfig(tile=tile)
             try:
                 run, result = _kernel_case(kind, M, K, B, activation, dtype, storage, cfg, g, dev)
@@ -172,7 +179,7 @@ def tune_kernels(dims, B: int, activation: str, dtype: torch.dtype, *, reps: int
             us = _time_us(run, reps, replays)
             if timer is not None:
                 us = timer(kind, M, K, tile, us)
-            if best is None or us < best[0]:
+            if best is None or us < best[0] * (AUTO_MARGIN if best[1].tile == -1 else 1.0):
                 best = (us, cfg)
         if best is not None:
             entries.append(TuningEntry(TuningKey(kind, M, K, B, activation, dt), best[1], best[0] / 1e3, False))
@@ -216,7 +223,7 @@ def _torch_step(x, w, act, alpha=1e-4, gamma=0.5):
 def tune_wide(dims, B: int, activation: str, dtype: torch.dtype, *, seed: int = 0, reps: int = 5, replays: int = 3,
               rejected: list | None = None, perturb=None, timer=None) -> dict | None:
     """Fastest passing tile configuration of each wide-path phase and k-split
-    ({"pred", "infer", "weight", "ksplit"}, -1 = default), or None when the
+    ({"pred", "infer", "weight", "ksplit"}, -1 = automatic), or None when the
     net does not take the wide path.  ``perturb(phase, cfg, model)`` (tests)
     may alter a candidate's state after its step; ``timer(phase, cfg, us)``
     may replace a measured time."""
@@ -238,10 +245,11 @@ def tune_wide(dims, B: int, activation: str, dtype: torch.dtype, *, seed: int = 
     del probe_model
 
     def candidates(phase):
-        n = int(nat.lib().ipc_plan_wide_config_count(phase, split))
+        # -1, the automatic choice (the only way to the 64 x 64 tiles), first: a tie keeps it
+        configs = range(-1, int(nat.lib().ipc_plan_wide_config_count(phase, split)))
         if phase == nat_phase("pred"):
-            return [(c, k) for c in range(n) for k in (-1, 1, 2, 4, 8, 16)]
-        return [(c, -1) for c in range(n)]
+            return [(c, k) for c in configs for k in (-1, 1, 2, 4, 8, 16)]
+        return [(c, -1) for c in configs]
 
     chosen = {"pred": -1, "infer": -1, "weight": -1, "ksplit": -1}
     for name in ("pred", "infer", "weight"):
@@ -271,7 +279,7 @@ def tune_wide(dims, B: int, activation: str, dtype: torch.dtype, *, seed: int = 
                           reps, replays)
             if timer is not None:
                 us = timer(name, (cfg, ks), us)
-            if best is None or us < best[0]:
+            if best is None or us < best[0] * (AUTO_MARGIN if best[1:] == (-1, -1) else 1.0):
                 best = (us, cfg, ks)
             del m
         if best is not None:

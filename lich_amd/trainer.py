@@ -80,7 +80,7 @@ class IPCConfig:
     # operands reach 0.5x the bar or beyond); 2 otherwise (the MFMA-bound
     # wide path).
     pred_split: int | None = None
-    # Wide path tile configuration (pred, infer, weight, ksplit), -1 = default
+    # Wide path tile configuration (pred, infer, weight, ksplit), -1 = automatic
     # (ipc_plan_set_wide_config); a policy file's tuned choice takes precedence.
     wide_config: tuple[int, int, int, int] | None = None
     # Layer-resident plans: rows of the top layer per workgroup (16, 32 or
