@@ -119,10 +119,11 @@ bool chunk_fits(const GemmProblem& q, int esize) {
 // 512, and 1024 on its 16 x 16 tiles, which few tiles take only).
 constexpr long long kMaxThreads = 1LL << 32;
 
-// Output tiles of edge `e` over `n` problems.
-long long count_tiles(const GemmProblem* q, int n, int e) {
+// Output tiles of edge E over `n` problems.
+template <int E>
+long long count_tiles(const GemmProblem* q, int n) {
   long long t = 0;
-  for (int i = 0; i < n; ++i) t += ((q[i].M + e - 1LL) / e) * ((q[i].N + e - 1LL) / e) * q[i].groups;
+  for (int i = 0; i < n; ++i) t += (long long)((q[i].M + E - 1u) / E) * ((q[i].N + E - 1u) / E) * q[i].groups;
   return t;
 }
 
@@ -155,7 +156,7 @@ bool use_chunk(const GemmProblem* q, int n, int esize, bool fp32_operands, int s
   }
   if (n == 0) return true;
   const bool infer = q[0].kind == KIND_INFER;
-  const long long t64 = count_tiles(q, n, 64);
+  const long long t64 = count_tiles<64>(q, n);
   if (t64 * 512 >= kMaxThreads) return false;
   if (t64 > 256 && kmax <= 128) return false;
   if (t64 > 512 && kmax <= (infer ? 256 : 512)) return false;
@@ -167,7 +168,7 @@ bool use_chunk(const GemmProblem* q, int n, int esize, bool fp32_operands, int s
     if (rows && (act == IPC_ACT_SIGMOID || act == IPC_ACT_SILU) && (esize == 4 || !full)) return false;
     if (rows && (act == IPC_ACT_TANH || act == IPC_ACT_GELU) && fp32_operands && !full) return false;
   }
-  return !(esize == 4 && !infer && kmax >= 1024 && count_tiles(q, n, 128) >= 512);
+  return !(esize == 4 && !infer && kmax >= 1024 && count_tiles<128>(q, n) >= 512);
 }
 
 // Tile of such a launch.  `tile`: IPC_TILE_AUTO, or a generic tile id: 32 x 32,
@@ -189,16 +190,16 @@ bool use_chunk(const GemmProblem* q, int n, int esize, bool fp32_operands, int s
 // on 32 x 32, 295 on 64 x 64, inference 298, 234; (10, 4096 x 2, 784) at B = 20 491,
 // 292; nine more nets of 300-20,000 wide layers and B = 17-4096 the same either way).
 int pick_tile(int tile, const GemmProblem* q, int n, bool chunk) {
-  const long long t64 = count_tiles(q, n, 64);
+  const long long t64 = count_tiles<64>(q, n);
   if (chunk) {
-    const long long t32 = count_tiles(q, n, 32);
+    const long long t32 = count_tiles<32>(q, n);
     if (tile == IPC_TILE_32x32) return t32 * 512 >= kMaxThreads ? TILE_CHUNK_64 : t32 >= 256 ? TILE_CHUNK_32 : TILE_CHUNK_16;
     if (tile == IPC_TILE_64x64) return t64 >= 192 ? TILE_CHUNK_64 : TILE_CHUNK_32;
     if (tile == IPC_TILE_128x128) return TILE_CHUNK_64;
     return t64 >= 192 ? TILE_CHUNK_64 : t32 >= 256 ? TILE_CHUNK_32 : TILE_CHUNK_16;
   }
   if (tile != IPC_TILE_AUTO) return tile;
-  return count_tiles(q, n, 128) >= 512 ? IPC_TILE_128x128 : t64 >= 64 ? IPC_TILE_64x64 : IPC_TILE_32x32;
+  return count_tiles<128>(q, n) >= 512 ? IPC_TILE_128x128 : t64 >= 64 ? IPC_TILE_64x64 : IPC_TILE_32x32;
 }
 
 int launch_rc(hipError_t err, const char* what) {
@@ -313,7 +314,7 @@ int s16_auto_config(long long M, long long N, long long groups) {
 // 2^31 bytes stay (weight update 1024 x 1024, B = 2^20, 39.8 ms against 71.6 on
 // the tile kernel).
 bool generic_before_dma(const GemmProblem& q) {
-  return count_tiles(&q, 1, 64) <= (q.kind == KIND_INFER ? 512 : 256) && chunk_fits(q, 2);
+  return count_tiles<64>(&q, 1) <= (q.kind == KIND_INFER ? 512 : 256) && chunk_fits(q, 2);
 }
 
 // Pre-activation of a standalone call's B operand (ipc_set_s16_preactivate):
@@ -465,17 +466,17 @@ bool ws_lent(int storage, int mode, int act, const GemmProblem& q, int tile, boo
 
 // A call on the generic kernels: with a workspace lent, B activated into it first
 // (the kernel is the one that runs without, whose bits the result has).
-int run_generic(GemmProblem q, int storage, int operand, int split, int tile, bool lent, void* workspace, void* stream,
-                const char* what) {
-  const int run = generic_tile(tile, q, storage, operand, split);
-  if (lent) {
-    TRY(launch_rc(launch_s16_activate(q.b, workspace, (long long)q.groups * q.b_gs, operand, q.act_b, (hipStream_t)stream),
-                  what));
-    q.b = workspace;
-    q.act_b = IPC_ACT_IDENTITY;
-    q.vec_b = vec_ok(workspace, q.ldb, 2);
-  }
-  return launch_rc(launch_gemm(&q, 1, storage, operand, split, run, (hipStream_t)stream), what);
+int run_generic(const GemmProblem& p, int storage, int operand, int split, int tile, bool lent, void* workspace,
+                void* stream, const char* what) {
+  const int run = generic_tile(tile, p, storage, operand, split);
+  hipStream_t s = (hipStream_t)stream;
+  if (!lent) return launch_rc(launch_gemm(&p, 1, storage, operand, split, run, s), what);
+  TRY(launch_rc(launch_s16_activate(p.b, workspace, (long long)p.groups * p.b_gs, operand, p.act_b, s), what));
+  GemmProblem q = p;
+  q.b = workspace;
+  q.act_b = IPC_ACT_IDENTITY;
+  q.vec_b = vec_ok(workspace, q.ldb, 2);
+  return launch_rc(launch_gemm(&q, 1, storage, operand, split, run, s), what);
 }
 
 int check_workspace(const void* workspace, long long ws_bytes) {
