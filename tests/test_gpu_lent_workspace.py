@@ -61,3 +61,28 @@ def test_lent_workspace_is_used_and_changes_no_bit(mode, M, K, B, groups, act, d
         assert (ki.workspace_bytes > 0) == (mode == 1 and 3 <= route < 16)
     finally:
         nat.lib().ipc_set_s16_preactivate(-1)
+
+
+def test_lent_workspace_under_graph_capture():
+    """Both launches of a k-chunk call with a workspace are recorded; replays, with
+    the workspace overwritten and eager calls in between, give the eager bits."""
+    M, K, B, dt = 1024, 1024, 1024, torch.float16
+    report("lent-workspace-graph")
+    g = gen(7)
+    xu, w, xl = (randn(s, g).to(dt).to(DEV) for s in ((K, B), (M, K), (M, B)))
+    w.mul_(K ** -0.5)
+    k = PredictionErrorKernel("p", M, K, B, "gelu", dt, None, None)
+    assert nat.lib().ipc_kernel_route(0, M, K, B, 1, nat.dtype_code(dt), nat.act_code("gelu"), -1) >= 16
+    ws, eager, out = k.new_workspace(), torch.zeros_like(xl), torch.zeros_like(xl)
+    k(xu, w, xl, eager)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=torch.cuda.Stream()):
+        k(xu, w, xl, out, workspace=ws)
+    for _ in range(3):
+        out.zero_()
+        ws.fill_(255)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, eager)
+        k(xu, w, xl, out)
+        assert torch.equal(out, eager)
